@@ -760,6 +760,41 @@ St LaunchFp8BlockGemm(const BlockGemmArgs& a) {
   const bool dense_ok = !a.moe && !a.a_gather && (a.out_kind == kOutBf16 || a.out_kind == kOutF32) &&
                         (contiguous1 || !a.check_codes) && (uint64_t)a.a_rows_total * a.k <= 0xffffffffull &&
                         (uint64_t)a.n * a.k <= 0xffffffffull;
+  // UE8M0 scales: tiles chosen per shape from one row up (gemm_tile.hip), in
+  // place of the small-M kernel and of the 128 x 256 tiles.  DeepSeek
+  // launch_fp8_gemm, K -> N, us before -> after (one MI355X, weights rotated
+  // past the caches), M 4 / 64 / 301 / 2048:
+  //   4096 -> 1024   5.8 -> 4.2    15.4 -> 4.8    28.6 -> 6.8    31 -> 15.4
+  //   1024 -> 32768  9.8 -> 7.4    15.0 -> 9.5    32.6 -> 24.1   134 -> 114
+  //   8192 -> 4096   10.9 -> 7.7   29.5 -> 12.4   50.2 -> 22.5   78 -> 80
+  //   4096 -> 2048   6.0 -> 4.8    15.5 -> 5.9    29.0 -> 9.2    34 -> 23.3
+  //   2048 -> 4096   5.0 -> 4.3    8.9 -> 5.6     18.4 -> 8.2    29.5 -> 27.3
+  if (dense_ok && a.scale_fmt == kScaleUe8m0) {
+    TileGemmArgs t;
+    t.a = a.a;
+    t.a_scale = static_cast<const uint8_t*>(a.a_scale);
+    t.w = a.w;
+    t.w_scale = static_cast<const uint8_t*>(a.w_scale);
+    t.out = a.out;
+    t.error_flag = a.error_flag;
+    t.stream = a.stream;
+    t.m = a.m;
+    t.n = a.n;
+    t.k = a.k;
+    t.problems = a.problems;
+    t.a_rows_total = a.a_rows_total;
+    t.a_row_stride = a.a_row_stride;
+    t.a_prob_row = a.a_prob_row;
+    t.out_row_stride = a.out_row_stride;
+    t.out_prob_col = a.out_prob_col;
+    t.out_kind = a.out_kind;
+    t.check_codes = a.check_codes;
+    t.err_code_bit = a.err_code_bit;
+    t.err_scale_bit = a.err_scale_bit;
+    t.err_nonfinite_bit = a.err_nonfinite_bit;
+    t.write_nonfinite = a.write_nonfinite;
+    if (TileGemmTakes(t)) return LaunchTileGemm(t);
+  }
   // Above 64 rows the big tiles also take what the 128 x 128 kernel took
   // before (more than 256 rows, or too many 128 x 128 tiles for the small-M
   // kernel) and the small-M kernel's 64-row chunks once together they would
@@ -965,6 +1000,35 @@ St LaunchBf16Gemm(const Bf16GemmArgs& a) {
   // 170 us, m = 64 177 us, m = 128 233 -> 186 us, m = 200 364 -> 285 us;
   // m = 1 stays on the GEMV, 159 us).
   const bool wide = a.m >= 2 && a.m < 256 && a.n % 128 == 0 && a.k % 64 == 0 && a.n / 256 >= 192;
+  // Tiles chosen per shape (gemm_tile.hip) from two rows up; one row, and
+  // very wide weights up to 128 rows (HBM-bound on the big tiles: 6.1 TB/s),
+  // stay where they are.  Qwen3-8B projections, K -> N, us before -> after at
+  // M 2 / 17 / 57 / 200 / 2048 (one MI355X, weights rotated past the caches):
+  //   4096 -> 4096   8.5 -> 7.8    10.9 -> 8.3   14.3 -> 11.3   25 -> 16   63 -> 57
+  //   4096 -> 1024   6.2 -> 6.1    9.1 -> 6.0    12.8 -> 6.1    21 -> 8.1  33 -> 28
+  //   4096 -> 12288  20.4 -> 16.5  21.9 -> 18.7  30.5 -> 21.3   47 -> 38   182 -> 165
+  //   12288 -> 4096  17.3 -> 17.7  23.5 -> 20.4  37 -> 29       48 -> 43   182 -> 160
+  // (above 64 rows only what was taken there: whole 128-column groups)
+  if (a.m >= 2 && (a.m <= 64 || a.n % 128 == 0) && (!wide || a.m > 128)) {
+    TileGemmArgs t;
+    t.a = a.a;
+    t.w = a.w;
+    t.out = a.out;
+    t.stream = a.stream;
+    t.m = a.m;
+    t.n = a.n;
+    t.k = a.k;
+    t.a_rows_total = a.m;
+    t.bf16 = true;
+    t.out_kind = a.out_kind;
+    if (a.error_flag && a.nonfinite_bit) {
+      t.error_flag = a.error_flag;
+      t.err_code_bit = t.err_scale_bit = 0u;
+      t.err_nonfinite_bit = a.nonfinite_bit;
+    }
+    t.write_nonfinite = true;
+    if (TileGemmTakes(t)) return LaunchTileGemm(t);
+  }
   if (a.m <= 64 && !wide) return LaunchBf16Gemv(a);
   if (a.n % 128 || a.k % 64) return Invalid("bf16_gemm_shape_invalid");
   if ((Bf16BigTiles(a.m, a.n, a.k) || wide) && (uint64_t)a.m * a.k * 2 <= 0xffffffffull &&

@@ -1,0 +1,868 @@
+// Dense GEMMs of mid-size batches for gfx950: out [m, n] = A [m, k] . W [n, k]^T
+// with bf16 operands, or e4m3 operands and UE8M0 scales (one per A row and
+// 128 k, one per 128 W rows and 128 k), fp32 accumulation.
+//
+// What bounds such a call: not HBM alone.  A block reads its A rows as well as
+// its W rows, and a CU takes in ~64 GB/s while part of its lines come from HBM
+// or the MALL (~100 GB/s when all hit L2; deeper rings, other row patterns,
+// staggered K orders and an L2 prefetch through the scalar cache did not raise
+// it), against the ~23 GB/s that is its share of HBM.  So a tile of TM x TN
+// costs a CU (TM + TN) x row bytes at that rate, and what matters is that all
+// 256 CUs have a tile and that TM + TN is no larger than that takes.  The
+// 128 x 256 tiles of gemm_fp8_moe.hip leave most CUs idle at these sizes, and
+// the 16-row GEMV blocks read all of A for every 16 weight rows in the waves'
+// own loads.  Here the tile is chosen per call (PickTile) from 16-row steps
+// both ways.  Figures: at the dispatch rules in gemm_mfma.hip.
+//
+// A block is 4 multiplying and 4 loading waves: a wave issues in order, and a
+// DMA that the full load queue does not take yet would hold back the MFMAs
+// behind it (one kind of wave doing both: 5-15 % slower).  A K step is 256
+// bytes of every tile row, moved into LDS by DMA (global_load_lds_dwordx4, 4
+// rows x 256 bytes an instruction, the same number from every loading wave),
+// kStages steps deep: one wait and one barrier a step.  16-byte chunk c of row r sits in slot c ^ (r & 15) of its 256
+// bytes, so that a fragment read (16 rows, one chunk each) covers the 64
+// banks once.  The multiplying waves split the step's K, not the tile: each reads its
+// share of every row, so an LDS byte is read once (bf16: four k quarters;
+// e4m3: two 128-k halves, times two halves of the W rows), and the waves'
+// sums meet in LDS at the end in a fixed order, from which whole output rows
+// are stored.  The MFMA's first operand is W, so a lane's four results are
+// four consecutive columns of one row.
+//
+// e4m3 NaN codes count as 0 and raise the code bit, as the reference decodes
+// them (plugins/kernels/deepseek-v4-sm89/native/deepseek_fp8_gemm.cu:11-70):
+// a code turns every sum over its row into a NaN, so an element that came out
+// non-finite looks for codes in its two operand rows and, finding one, is
+// summed again the reference's way.  A 0xFF scale's block adds nothing.
+#include <algorithm>
+#include <type_traits>
+
+#include "device_common.hpp"
+#include "kernels.hpp"
+
+namespace pih_amd {
+namespace {
+
+enum : int { kTileBf16 = 0, kTileFp8 = 1 };
+constexpr uint32_t SB = 256;  // bytes of a row per K step
+constexpr uint32_t kGridStep = 128;  // ... in the kernel that walks tiles
+constexpr uint32_t kCus = 256;
+constexpr uint32_t kThreads = 512;  // waves 0-3 multiply, waves 4-7 load
+constexpr uint32_t kMaxKb = 64;  // e4m3: K / 128 the scale panels hold
+constexpr uint32_t kOutPitch = 144;  // staged output rows: 128 bytes + 16
+// bytes between the blocks of the waves' sums: the four 16-lane groups 16
+// bytes off a bank period, so that a row's columns are read without conflicts
+constexpr uint32_t kSumGroup = 272, kSumBlock = 4 * kSumGroup;
+
+struct TileParams {
+  const uint8_t* a;
+  const uint8_t* w;
+  const uint8_t* a_scale;
+  const uint8_t* w_scale;
+  void* out;
+  uint32_t* err;
+  uint32_t m, n, row_bytes, m_tiles, n_tiles, problems;
+  uint32_t a_row_stride, a_prob_row;
+  uint64_t out_row_stride;
+  uint32_t out_prob_col;
+  uint32_t out_f32, write_nonfinite, check_codes;
+  uint32_t err_code, err_scale, err_nonfinite;
+};
+
+typedef unsigned int v4u __attribute__((ext_vector_type(4)));
+
+__device__ __forceinline__ const uint8_t* uniform_ptr(const uint8_t* p) {
+  const uint64_t v = reinterpret_cast<uint64_t>(p);
+  const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v), hi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
+  return reinterpret_cast<const uint8_t*>(((uint64_t)hi << 32) | lo);
+}
+
+// s_waitcnt immediates: vmcnt <= n (n < 64) alone; every LDS read returned
+// (the stage a wave has read may be refilled once all are past the barrier)
+constexpr int vmcnt_at_most(int n) { return ((n >> 4) << 14) | 0x0F70 | (n & 15); }
+constexpr int kLdsRead = 0xC07F;
+
+// Output element (A row ar, column col of problem prob) the reference's way:
+// per 128-k block an fp32 sum of decoded e4m3 products in k order with NaN
+// codes as 0, a block with a 0xFF scale skipped before it is read.  False
+// when neither operand row holds a code.  (Loops kept rolled: this is rare,
+// and code in the way of the common path costs instruction fetches.)
+__device__ __forceinline__ bool code_element(const TileParams& p, uint64_t ar, uint32_t prob, uint32_t col, float& sum,
+                                             uint32_t& bits) {
+  const uint32_t RB = p.row_bytes, KB = RB / 128;
+  const uint8_t* ap = p.a + ar * RB;
+  const uint8_t* wp = p.w + ((uint64_t)prob * p.n + col) * RB;
+  const uint8_t* asp = p.a_scale + ar * KB;
+  const uint8_t* wsp = p.w_scale + ((uint64_t)prob * (p.n / 128) + col / 128) * KB;
+  uint32_t any = 0;
+  sum = 0.0f;
+  bits = 0;
+#pragma unroll 1
+  for (uint32_t b = 0; b < KB; ++b) {
+    const bool skip = asp[b] == 0xffu || wsp[b] == 0xffu;
+    if (skip) bits |= kErrScale;
+    float local = 0.0f;
+#pragma unroll 1
+    for (uint32_t c = b * 128; c < b * 128 + 128; c += 4) {
+      const uint32_t x = *reinterpret_cast<const uint32_t*>(ap + c), y = *reinterpret_cast<const uint32_t*>(wp + c);
+      const uint32_t nx = e4m3_nan_bytes(x), ny = e4m3_nan_bytes(y);
+      any |= nx | ny;
+      if ((nx | ny) && !skip) bits |= kErrCode;
+      const uint32_t xa = e4m3_nan_to_zero(x, nx), xw = e4m3_nan_to_zero(y, ny);
+#pragma unroll 1
+      for (uint32_t e = 0; e < 32; e += 8) local = local + e4m3_decode((xa >> e) & 0xffu) * e4m3_decode((xw >> e) & 0xffu);
+    }
+    if (!skip) sum = sum + local * ue8m0_value(asp[b]) * ue8m0_value(wsp[b]);
+  }
+  return any != 0;
+}
+
+__device__ __forceinline__ bool finite4(v4f v) {
+  return __builtin_isfinite(v[0]) && __builtin_isfinite(v[1]) && __builtin_isfinite(v[2]) && __builtin_isfinite(v[3]);
+}
+
+// four columns from `col` of output row `row`, or one of them
+__device__ __forceinline__ void store4(const TileParams& p, uint32_t row, uint32_t prob, uint32_t col, v4f v) {
+  const uint64_t o = (uint64_t)row * p.out_row_stride + (uint64_t)prob * p.out_prob_col + col;
+  if (p.out_f32) *reinterpret_cast<v4f*>(static_cast<float*>(p.out) + o) = v;
+  else
+    *reinterpret_cast<uint2*>(static_cast<uint16_t*>(p.out) + o) =
+        uint2{f32x2_to_bf16x2(v[0], v[1]), f32x2_to_bf16x2(v[2], v[3])};
+}
+__device__ __forceinline__ void store1(const TileParams& p, uint32_t row, uint32_t prob, uint32_t col, float v) {
+  const uint64_t o = (uint64_t)row * p.out_row_stride + (uint64_t)prob * p.out_prob_col + col;
+  if (p.out_f32) static_cast<float*>(p.out)[o] = v;
+  else static_cast<uint16_t*>(p.out)[o] = (uint16_t)f32_to_bf16_bits(v);
+}
+
+// The non-finite element v at (row, col): e4m3 operands that hold a NaN code
+// get the reference's sum and its bits; otherwise the value stays and raises
+// the non-finite bit, stored unless the caller leaves such elements out.
+template <int OP>
+__device__ __forceinline__ void store_nonfinite(const TileParams& p, uint32_t row, uint32_t prob, uint32_t col, float v,
+                                                uint32_t& bad) {
+  if (OP == kTileFp8 && p.check_codes) {
+    float sum;
+    uint32_t bits;
+    if (code_element(p, (uint64_t)row * p.a_row_stride + (uint64_t)prob * p.a_prob_row, prob, col, sum, bits)) {
+      v = sum;
+      bad |= bits;
+    }
+  }
+  const bool fin = __builtin_isfinite(v);
+  if (!fin) bad |= kErrNonFinite;
+  if (fin || !p.err_nonfinite || p.write_nonfinite) store1(p, row, prob, col, v);
+}
+
+__device__ __forceinline__ void raise(const TileParams& p, uint32_t bad) {
+  const uint32_t bits = ((bad & kErrCode) ? p.err_code : 0u) | ((bad & kErrScale) ? p.err_scale : 0u) |
+                        ((bad & kErrNonFinite) ? p.err_nonfinite : 0u);
+  if (bits) atomicOr(p.err, bits);
+}
+
+__device__ __forceinline__ uint32_t has_ff(uint32_t v) { return (~v - 0x01010101u) & v & 0x80808080u; }
+
+template <int OP, int MB, int NB>
+struct TileShape {
+  static constexpr uint32_t TM = 16 * MB, TN = 16 * NB, kStage = (TM + TN) * SB;
+  // 256 bytes of W scales and TM x kMaxKb of A scales, each in whole DMAs
+  static constexpr uint32_t kPanel = OP == kTileFp8 ? 256 + TM * kMaxKb : 0;
+  static constexpr uint32_t kLds = 160 * 1024 - 512;
+  static constexpr int kLoads = MB + NB;  // DMAs per wave and step
+  static constexpr int kFit = (int)((kLds - kPanel) / kStage);
+  // as deep as LDS allows, at most 8 steps and 63 loads in flight
+  static constexpr int kStages = std::min(std::min(kFit, 8), 63 / kLoads + 1);
+  static constexpr int kParts = OP == kTileFp8 ? 2 : 4;  // waves that share an output
+  static constexpr uint32_t kSums = kParts * MB * NB * kSumBlock;
+  static constexpr uint32_t kRing = kStages * kStage > kSums ? kStages * kStage : kSums;
+};
+
+template <int OP, int MB, int NB>
+__global__ __launch_bounds__(kThreads, 1) void tile_gemm_kernel(TileParams p) {
+  using S = TileShape<OP, MB, NB>;
+  constexpr uint32_t TM = S::TM, TN = S::TN;
+  constexpr int ST = S::kStages, NL = S::kLoads;
+  static_assert(ST >= 2, "two stages");
+  constexpr bool kFp8 = OP == kTileFp8;
+  // e4m3: the two wave pairs take half of the W blocks each, or of the A
+  // blocks; with an odd number of both one pair does all (the loads bound it)
+  constexpr bool kSplitN = kFp8 && NB % 2 == 0, kSplitM = kFp8 && !kSplitN && MB % 2 == 0;
+  constexpr bool kOnePair = kFp8 && !kSplitN && !kSplitM;
+  constexpr int MW = kSplitM ? MB / 2 : MB, NW = kSplitN ? NB / 2 : NB;  // a wave's blocks
+  __shared__ __align__(16) uint8_t smem[S::kRing + S::kPanel];
+  const uint32_t tid = threadIdx.x, lane = tid & 63, lr = lane & 15, lg = lane >> 4;
+  const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6), wv = wave & 3;
+  const bool loader = wave >= 4;
+  const uint32_t lds0 = lds_addr(smem);
+
+  // tile t of (problem, N tile, M tile), M fastest: the tiles that share W
+  // rows run side by side on one XCD, which walks a contiguous range
+  const uint32_t total = p.m_tiles * p.n_tiles * p.problems, per = (total + 7) / 8;
+  const uint32_t t = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
+  if ((blockIdx.x >> 3) >= per || t >= total) return;
+  const uint32_t mt = t % p.m_tiles, rest = t / p.m_tiles, nt = rest % p.n_tiles, prob = rest / p.n_tiles;
+  const uint32_t row0 = mt * TM, col0 = nt * TN;
+  const uint32_t RB = p.row_bytes, steps = RB / SB;
+  uint32_t bad = 0;
+
+  // tile rows past m read row m - 1; they are not stored
+  auto a_row = [&](uint32_t r) -> uint64_t {
+    return (uint64_t)min(row0 + r, p.m - 1) * p.a_row_stride + (uint64_t)prob * p.a_prob_row;
+  };
+  const uint8_t* const w_base = p.w + ((uint64_t)prob * p.n + col0) * RB;
+
+  // ---- DMA sources: instruction i of wave w moves rows 16 i + 4 w + (l >> 4),
+  // lane l's 16 bytes to slot l & 15 (chunk (l & 15) ^ (row & 15))
+  const uint32_t drow = 4 * wv + lg, dchunk = (lr ^ drow) << 4;
+  uint32_t a_off[MB], w_off[NB];
+#pragma unroll
+  for (int i = 0; i < MB; ++i) a_off[i] = (uint32_t)(a_row(16 * i + drow) * RB) + dchunk;
+#pragma unroll
+  for (int i = 0; i < NB; ++i) w_off[i] = (16 * i + drow) * RB + dchunk;
+  auto issue = [&](uint32_t stage, uint32_t j, auto NT) __attribute__((always_inline)) {
+    const uint32_t lds = lds0 + stage * S::kStage + wv * 1024;
+    const uint8_t* ab = uniform_ptr(p.a + (uint64_t)j * SB);
+    const uint8_t* wb = uniform_ptr(w_base + (uint64_t)j * SB);
+#pragma unroll
+    for (int i = 0; i < NB; ++i) {
+      if constexpr (decltype(NT)::value) dma16nt(wb, w_off[i], lds + TM * SB + i * 4096);
+      else dma16(wb, w_off[i], lds + TM * SB + i * 4096);
+    }
+#pragma unroll
+    for (int i = 0; i < MB; ++i) dma16(ab, a_off[i], lds + i * 4096);
+  };
+
+  // ---- e4m3: the tile's scales, whole panels by dword DMA ahead of the
+  // first step: KB bytes of W scales, TM rows of KB bytes of A scales
+  const uint32_t KB = RB / 128;  // e4m3 only
+  const uint8_t* const pw = smem + S::kRing;
+  const uint8_t* const pa = pw + 256;
+  if (kFp8 && loader) {
+    const uint32_t q4 = KB / 4;  // dwords per row (the launcher checks KB % 4)
+    if (wv == 0) {
+      const uint8_t* src = p.w_scale + ((uint64_t)prob * (p.n / 128) + col0 / 128) * KB;
+      dma4v(src + 4 * min(lane, q4 - 1), lds0 + S::kRing);
+    }
+    for (uint32_t b = wv * 64; b < TM * q4; b += 256) {
+      const uint32_t i = min(b + lane, TM * q4 - 1);
+      dma4v(p.a_scale + a_row(i / q4) * KB + 4 * (i % q4), lds0 + S::kRing + 256 + 4 * b);
+    }
+  }
+
+  // a wave's accumulators [W block][A block]
+  v4f acc[NW][MW];
+#pragma unroll
+  for (int n = 0; n < NW; ++n)
+#pragma unroll
+    for (int r = 0; r < MW; ++r) acc[n][r] = v4f{0.f, 0.f, 0.f, 0.f};
+  const uint32_t kh = wv & 1, half = wv >> 1;
+  const uint32_t mb0 = kSplitM ? half * MW : 0, nb0 = kSplitN ? half * NW : 0;
+
+  auto compute = [&](uint32_t stage, uint32_t j, auto FF) __attribute__((always_inline)) {
+    if (kOnePair && half) return;
+    const uint8_t* sa = smem + stage * S::kStage + (mb0 * 16 + lr) * SB;
+    const uint8_t* sw = smem + stage * S::kStage + (TM + nb0 * 16 + lr) * SB;
+    if constexpr (!kFp8) {
+      const uint32_t at = ((4 * wv + lg) ^ lr) << 4;
+      v4i wf[NW];
+#pragma unroll
+      for (int n = 0; n < NW; ++n) wf[n] = *reinterpret_cast<const v4i*>(sw + n * 4096 + at);
+#pragma unroll
+      for (int r = 0; r < MW; ++r) {
+        const v4i af = *reinterpret_cast<const v4i*>(sa + r * 4096 + at);
+#pragma unroll
+        for (int n = 0; n < NW; ++n)
+          acc[n][r] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8bf, wf[n]),
+                                                              __builtin_bit_cast(v8bf, af), acc[n][r], 0, 0, 0);
+      }
+    } else {
+      const uint32_t at0 = ((8 * kh + lg) ^ lr) << 4, at1 = ((8 * kh + 4 + lg) ^ lr) << 4;
+      auto frag = [&](const uint8_t* s) __attribute__((always_inline)) -> v8i {
+        const v4i x = *reinterpret_cast<const v4i*>(s + at0), y = *reinterpret_cast<const v4i*>(s + at1);
+        return v8i{x[0], x[1], x[2], x[3], y[0], y[1], y[2], y[3]};
+      };
+      const uint32_t kb = 2 * j + kh;
+      uint32_t ws = pw[kb];
+      const bool wff = decltype(FF)::value && ws == 0xffu;
+      if (wff) ws = 0;
+      v8i wf[NW];
+#pragma unroll
+      for (int n = 0; n < NW; ++n) wf[n] = frag(sw + n * 4096);
+#pragma unroll
+      for (int r = 0; r < MW; ++r) {
+        v8i af = frag(sa + r * 4096);
+        uint32_t as = pa[(mb0 * 16 + r * 16 + lr) * KB + kb];
+        if constexpr (decltype(FF)::value) {
+          // a 0xFF scale's block adds nothing: an A row's fragment becomes 0;
+          // a W block runs with both scales 0 (2^-254 times a sum below 2^25
+          // is below the fp32 range)
+          const int keep = as == 0xffu ? 0 : -1;
+#pragma unroll
+          for (int q = 0; q < 8; ++q) af[q] &= keep;
+          as = as == 0xffu ? 127u : as;
+          as = wff ? 0u : as;
+        }
+#pragma unroll
+        for (int n = 0; n < NW; ++n)
+          acc[n][r] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(wf[n], af, acc[n][r], 0, 0, 0, (int)ws, 0,
+                                                                       (int)as);
+      }
+    }
+  };
+
+  // ---- the K loop: ST stages.  A loading wave waits for its part of step
+  // j's stage, meets the others at the barrier and sends for step j + ST - 1
+  // (the last ST - 1 steps send for nothing and wait for less each); a
+  // multiplying wave meets the barrier and multiplies step j.
+  const uint32_t lead = min((uint32_t)(ST - 1), steps);
+  auto tail_wait = [&](int left) __attribute__((always_inline)) {
+    // `left` further steps are in flight
+#define PIH_TILE_WAIT(L) \
+  case L:                \
+    if constexpr ((L) < ST - 1) __builtin_amdgcn_s_waitcnt(vmcnt_at_most((L) * NL)); \
+    break;
+    switch (left) {
+      PIH_TILE_WAIT(0) PIH_TILE_WAIT(1) PIH_TILE_WAIT(2) PIH_TILE_WAIT(3)
+      PIH_TILE_WAIT(4) PIH_TILE_WAIT(5) PIH_TILE_WAIT(6)
+    }
+#undef PIH_TILE_WAIT
+  };
+  auto load_loop = [&](auto NT) __attribute__((always_inline)) {
+#pragma unroll
+    for (int s = 0; s < ST - 1; ++s)
+      if ((uint32_t)s < lead) issue(s, s, NT);
+    if constexpr (kFp8) {
+      // the scale panels are older loads than the stages'
+      if (lead == ST - 1) __builtin_amdgcn_s_waitcnt(vmcnt_at_most((ST - 1) * NL));
+      else __builtin_amdgcn_s_waitcnt(vmcnt_at_most(0));
+      __builtin_amdgcn_s_barrier();
+    }
+    uint32_t j = 0, ist = ST - 1;
+    for (; j + (ST - 1) < steps; ++j) {
+      __builtin_amdgcn_s_waitcnt(vmcnt_at_most((ST - 2) * NL));
+      __builtin_amdgcn_s_barrier();
+      issue(ist, j + (ST - 1), NT);
+      ist = ist + 1 == ST ? 0 : ist + 1;
+    }
+#pragma unroll
+    for (int left = ST - 2; left >= 0; --left) {
+      if (j + left >= steps) continue;  // fewer steps than stages
+      tail_wait(left);
+      __builtin_amdgcn_s_barrier();
+      ++j;
+    }
+  };
+  auto multiply_loop = [&](auto FF) __attribute__((always_inline)) {
+    uint32_t cst = 0;
+    for (uint32_t j = 0; j < steps; ++j) {
+      __builtin_amdgcn_s_waitcnt(kLdsRead);
+      __builtin_amdgcn_s_barrier();
+      compute(cst, j, FF);
+      cst = cst + 1 == ST ? 0 : cst + 1;
+    }
+  };
+  if (loader) {
+    // one M tile reads each weight byte once: non-temporal, so that the A
+    // rows every tile reads again stay in L2
+    if (p.m_tiles == 1) load_loop(std::true_type{});
+    else load_loop(std::false_type{});
+  } else {
+    bool ff = false;
+    if constexpr (kFp8) {
+      // a 0xFF scale anywhere in the panels; every wave looks through all of
+      // them, which needs no exchange
+      __builtin_amdgcn_s_barrier();
+      uint32_t hit = 0;
+      for (uint32_t i = lane; i < TM * KB / 16; i += 64) {
+        const v4u v = reinterpret_cast<const v4u*>(pa)[i];
+        hit |= has_ff(v.x) | has_ff(v.y) | has_ff(v.z) | has_ff(v.w);
+      }
+      if (lane < KB / 4) hit |= has_ff(reinterpret_cast<const uint32_t*>(pw)[lane]);
+      ff = __builtin_amdgcn_ballot_w64(hit != 0) != 0;
+      if (ff) bad |= kErrScale;
+    }
+    if (kFp8 && ff) multiply_loop(std::true_type{});
+    else multiply_loop(std::false_type{});
+  }
+
+  // ---- the waves' sums, then whole rows
+  __syncthreads();
+  const uint32_t part = kFp8 ? kh : wv;
+#pragma unroll
+  for (int n = 0; n < NW && !loader && !(kOnePair && half); ++n)
+#pragma unroll
+    for (int r = 0; r < MW; ++r)
+      *reinterpret_cast<v4f*>(smem + (part * MB * NB + (mb0 + r) * NB + nb0 + n) * kSumBlock + lg * kSumGroup + lr * 16) =
+          acc[n][r];
+  __syncthreads();
+  constexpr uint32_t QR = TN / 4;  // 4-column groups per row
+#pragma unroll 1
+  for (uint32_t it = tid; it < TM * QR; it += kThreads) {
+    const uint32_t row = it / QR, cq = it % QR;
+    if (row0 + row >= p.m) continue;
+    const uint8_t* s = smem + ((row >> 4) * NB + (cq >> 2)) * kSumBlock + (cq & 3) * kSumGroup + (row & 15) * 16;
+    v4f v = *reinterpret_cast<const v4f*>(s);
+#pragma unroll
+    for (int q = 1; q < S::kParts; ++q) v += *reinterpret_cast<const v4f*>(s + q * MB * NB * kSumBlock);
+    if (finite4(v)) {
+      store4(p, row0 + row, prob, col0 + cq * 4, v);
+    } else {
+#pragma unroll 1
+      for (int i = 0; i < 4; ++i) {
+        const float e = i == 0 ? v[0] : i == 1 ? v[1] : i == 2 ? v[2] : v[3];
+        if (__builtin_isfinite(e)) store1(p, row0 + row, prob, col0 + cq * 4 + i, e);
+        else store_nonfinite<OP>(p, row0 + row, prob, col0 + cq * 4 + i, e, bad);
+      }
+    }
+  }
+  if (bad) raise(p, bad);
+}
+
+// ------------------------------------------------ several tiles per CU
+// The same operands and loading waves, for shapes of more tiles than CUs: a
+// block per CU walks its tiles, and the four multiplying waves take a quarter
+// of the tile each (2 x 2), so that nothing has to be summed across them: a
+// wave stores its results from its registers and goes on, while the loading
+// waves are already kStages - 1 steps into the next tile.  One barrier per K
+// step for all waves, none per tile.
+template <int OP, int MB, int NB, int SBW>
+struct GridShape {
+  static constexpr uint32_t TM = 16 * MB, TN = 16 * NB, kStage = (TM + TN) * SBW;
+  static constexpr uint32_t kPanelOne = OP == kTileFp8 ? 256 + TM * kMaxKb : 0;  // two of them
+  static constexpr uint32_t kLds = 160 * 1024 - 512;
+  static constexpr int kLoads = (MB + NB) * (int)SBW / 256;
+  static constexpr uint32_t kOut = 4 * 16 * kOutPitch;  // a 16-row x 128-byte piece of output per wave
+  static constexpr int kFit = (int)((kLds - 2 * kPanelOne - kOut) / kStage);
+  static constexpr int kStages = std::min(std::min(kFit, 8), 63 / kLoads + 1);
+  // fragments read ahead of their MFMAs; an e4m3 fragment is 8 registers, and
+  // three of them ahead spilled (128 x 128 tiles: 23.3 -> 25.5 us at M 2048,
+  // 4096 -> 2048; bf16 256 x 128: 60.6 -> 57.2 us at 4096 -> 4096 with three)
+  static constexpr int kAhead = OP == kTileBf16 ? 3 : 1;
+};
+
+template <int OP, int MB, int NB, int SBW>
+__global__ __launch_bounds__(kThreads, 1) void tile_grid_kernel(TileParams p) {
+  using S = GridShape<OP, MB, NB, SBW>;
+  constexpr uint32_t TM = S::TM, TN = S::TN;
+  constexpr int ST = S::kStages, NL = S::kLoads;
+  static_assert(ST >= 2 && MB % 2 == 0 && NB == 8 && ((MB + NB) * SBW) % 256 == 0, "shape");
+  constexpr bool kFp8 = OP == kTileFp8;
+  constexpr int MW = MB / 2, NW = NB / 2;
+  constexpr int RPI = 1024 / SBW, IPB = 16 / RPI;  // rows per DMA instruction, instructions per 16 rows (all waves)
+  __shared__ __align__(16) uint8_t smem[ST * S::kStage + 2 * S::kPanelOne + S::kOut];
+  const uint32_t tid = threadIdx.x, lane = tid & 63, lr = lane & 15, lg = lane >> 4;
+  const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6), wv = wave & 3;
+  const uint32_t lds0 = lds_addr(smem);
+  const uint32_t RB = p.row_bytes, steps = RB / SBW, KB = RB / 128;
+  const uint32_t total = p.m_tiles * p.n_tiles * p.problems, per = (total + 7) / 8;
+  const uint32_t xcd = blockIdx.x & 7, jstep = gridDim.x >> 3;
+  const uint32_t t_end = min((xcd + 1) * per, total);
+  const uint32_t t_first = xcd * per + (blockIdx.x >> 3);
+  if (t_first >= t_end) return;
+  const uint32_t tiles = (t_end - t_first + jstep - 1) / jstep;
+  auto tile_at = [&](uint32_t i, uint32_t& row0, uint32_t& col0, uint32_t& prob) __attribute__((always_inline)) {
+    const uint32_t t = t_first + i * jstep, mt = t % p.m_tiles, rest = t / p.m_tiles;
+    row0 = mt * TM;
+    col0 = (rest % p.n_tiles) * TN;
+    prob = rest / p.n_tiles;
+  };
+
+  if (wave >= 4) {
+    // ---- loading waves.  Instruction q of wave w moves rows
+    // RPI (4 q + w) + (l / (64 / RPI)) of the A rows followed by the W rows.
+    constexpr uint32_t LPR = 64 / RPI;
+    const uint32_t lrow = lane / LPR, lchunk = lane % LPR;
+    uint32_t off[NL];
+    const uint8_t* w_base = nullptr;
+    uint32_t li = 0, lj = 0, ist = 0;  // next load: tile, step, stage
+    static_assert((MB * IPB) % 4 == 0 && (NB * IPB) % 4 == 0, "every wave the same loads");
+    constexpr int NLA = MB * IPB / 4;
+    auto issue_next = [&]() __attribute__((always_inline)) {
+      if (lj == 0) {
+        uint32_t row0, col0, prob;
+        tile_at(li, row0, col0, prob);
+        w_base = p.w + ((uint64_t)prob * p.n + col0) * RB;
+        auto a_row = [&](uint32_t r) -> uint64_t {
+          return (uint64_t)min(row0 + r, p.m - 1) * p.a_row_stride + (uint64_t)prob * p.a_prob_row;
+        };
+#pragma unroll
+        for (int q = 0; q < NL; ++q) {
+          const uint32_t r = RPI * (4 * (q < NLA ? q : q - NLA) + wv) + lrow;
+          const uint32_t c = SBW == 256 ? lchunk ^ (r & 15) : lchunk ^ ((r >> 1) & 7);
+          off[q] = (q < NLA ? (uint32_t)(a_row(r) * RB) : r * RB) + (c << 4);
+        }
+        if constexpr (kFp8) {
+          const uint32_t q4 = KB / 4, pan = lds0 + ST * S::kStage + (li & 1) * S::kPanelOne;
+          if (wv == 0) {
+            const uint8_t* src = p.w_scale + ((uint64_t)prob * (p.n / 128) + col0 / 128) * KB;
+            dma4v(src + 4 * min(lane, q4 - 1), pan);
+          }
+          for (uint32_t b = wv * 64; b < TM * q4; b += 256) {
+            const uint32_t i = min(b + lane, TM * q4 - 1);
+            dma4v(p.a_scale + a_row(i / q4) * KB + 4 * (i % q4), pan + 256 + 4 * b);
+          }
+        }
+      }
+      const uint32_t lds = lds0 + ist * S::kStage + wv * 1024;
+      const uint8_t* ab = uniform_ptr(p.a + (uint64_t)lj * SBW);
+      const uint8_t* wb = uniform_ptr(w_base + (uint64_t)lj * SBW);
+#pragma unroll
+      for (int q = 0; q < NL; ++q) dma16(q < NLA ? ab : wb, off[q], lds + q * 4096);
+      ist = ist + 1 == ST ? 0 : ist + 1;
+      if (++lj == steps) {
+        lj = 0;
+        ++li;
+      }
+    };
+    const uint32_t all = tiles * steps;
+#pragma unroll 1
+    for (uint32_t s = 0; s < min((uint32_t)(ST - 1), all); ++s) issue_next();
+    uint32_t g = 0;
+    for (; g + (ST - 1) < all; ++g) {
+      __builtin_amdgcn_s_waitcnt(vmcnt_at_most((ST - 2) * NL));
+      __builtin_amdgcn_s_barrier();
+      issue_next();
+    }
+#pragma unroll
+    for (int left = ST - 2; left >= 0; --left) {
+      if (g + left >= all) continue;
+      switch (left) {
+#define PIH_TILE_WAIT(L) \
+  case L:                \
+    if constexpr ((L) < ST - 1) __builtin_amdgcn_s_waitcnt(vmcnt_at_most((L) * NL)); \
+    break;
+        PIH_TILE_WAIT(0) PIH_TILE_WAIT(1) PIH_TILE_WAIT(2) PIH_TILE_WAIT(3)
+        PIH_TILE_WAIT(4) PIH_TILE_WAIT(5) PIH_TILE_WAIT(6)
+#undef PIH_TILE_WAIT
+      }
+      __builtin_amdgcn_s_barrier();
+      ++g;
+    }
+    __builtin_amdgcn_s_barrier();  // the multiplying waves' look past the last step
+    return;
+  }
+
+  // ---- multiplying waves.  A step is GS groups of one A fragment times the
+  // wave's NW W fragments of its K slice (32 bf16 or 128 e4m3 values); A
+  // fragments are read kAhead groups ahead and W fragments a slice ahead, over
+  // the step's end: the barrier that opens step j + 1 stands kAhead groups
+  // before the end of step j, when every fragment of step j is in registers.
+  const uint32_t wm = wv >> 1, wn = wv & 1;
+  uint32_t bad = 0, cst = 0;
+  constexpr int QS = kFp8 ? SBW / 128 : SBW / 64, GS = QS * MW;
+  constexpr int D = S::kAhead, AR = D + 1;
+  static_assert(D <= MW && GS % AR == 0, "fragment ring");
+  using Frag = std::conditional_t<kFp8, v8i, v4i>;
+  Frag af[AR], wf[2][NW];
+  uint32_t as[AR], ws[2];
+  const uint32_t a_lane = (wm * MW * 16 + lr) * SBW, w_lane = (TM + wn * NW * 16 + lr) * SBW;
+  auto frag = [&](const uint8_t* s, int q) __attribute__((always_inline)) -> Frag {
+    auto at = [&](uint32_t c) -> uint32_t { return (SBW == 256 ? c ^ lr : c ^ (lr >> 1)) << 4; };
+    if constexpr (kFp8) {
+      const v4i x = *reinterpret_cast<const v4i*>(s + at(8 * q + lg)), y = *reinterpret_cast<const v4i*>(s + at(8 * q + 4 + lg));
+      return v8i{x[0], x[1], x[2], x[3], y[0], y[1], y[2], y[3]};
+    } else {
+      return *reinterpret_cast<const v4i*>(s + at(4 * q + lg));
+    }
+  };
+  auto read_a = [&](uint32_t stage, uint32_t j, const uint8_t* pan, int g, int slot) __attribute__((always_inline)) {
+    const int r = g % MW, q = g / MW;
+    af[slot] = frag(smem + stage * S::kStage + a_lane + r * 16 * SBW, q);
+    if constexpr (kFp8) as[slot] = pan[256 + ((wm * MW + r) * 16 + lr) * KB + j * QS + q];
+  };
+  auto read_w = [&](uint32_t stage, uint32_t j, const uint8_t* pan, int q, int buf) __attribute__((always_inline)) {
+#pragma unroll
+    for (int n = 0; n < NW; ++n) wf[buf][n] = frag(smem + stage * S::kStage + w_lane + n * 16 * SBW, q);
+    if constexpr (kFp8) ws[buf] = pan[j * QS + q];
+  };
+  const uint8_t* const panels = smem + ST * S::kStage;
+  __builtin_amdgcn_s_barrier();
+  read_w(0, 0, panels, 0, 0);
+#pragma unroll
+  for (int g = 0; g < D; ++g) read_a(0, 0, panels, g, g);
+  for (uint32_t i = 0; i < tiles; ++i) {
+    uint32_t row0, col0, prob;
+    tile_at(i, row0, col0, prob);
+    v4f acc[NW][MW];
+#pragma unroll
+    for (int n = 0; n < NW; ++n)
+#pragma unroll
+      for (int r = 0; r < MW; ++r) acc[n][r] = v4f{0.f, 0.f, 0.f, 0.f};
+    const uint8_t* const pan = panels + (i & 1) * S::kPanelOne;
+    // step j, whose first slice's W fragments are in wf[P]
+    auto step = [&](uint32_t j, auto PAR, auto FF) __attribute__((always_inline)) {
+      constexpr int P = decltype(PAR)::value;
+      const uint32_t nst = cst + 1 == ST ? 0 : cst + 1;
+      const bool wrap = j + 1 == steps;
+      const uint32_t nj = wrap ? 0 : j + 1;
+      const uint8_t* const npan = wrap ? panels + ((i + 1) & 1) * S::kPanelOne : pan;
+#pragma unroll
+      for (int g = 0; g < GS; ++g) {
+        const int r = g % MW, q = g / MW, wb = (P + q) & 1;
+        if (g != GS - D) {
+          if (g < GS - D) read_a(cst, j, pan, g + D, (g + D) % AR);
+          else read_a(nst, nj, npan, g + D - GS, (g + D) % AR);
+          if (q + 1 < QS && r == MW - D) read_w(cst, j, pan, q + 1, wb ^ 1);
+        }
+        Frag a = af[g % AR];
+        uint32_t sa = as[g % AR], sw = ws[wb];
+        if constexpr (kFp8 && decltype(FF)::value) {
+          // a 0xFF scale's block adds nothing (see compute above)
+          const int keep = sa == 0xffu ? 0 : -1;
+#pragma unroll
+          for (int e = 0; e < 8; ++e) a[e] &= keep;
+          const bool wff = sw == 0xffu;
+          sa = wff ? 0u : sa == 0xffu ? 127u : sa;
+          sw = wff ? 0u : sw;
+        }
+#pragma unroll
+        for (int n = 0; n < NW; ++n) {
+          if constexpr (kFp8)
+            acc[n][r] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(wf[wb][n], a, acc[n][r], 0, 0, 0, (int)sw, 0,
+                                                                         (int)sa);
+          else
+            acc[n][r] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8bf, wf[wb][n]),
+                                                                __builtin_bit_cast(v8bf, a), acc[n][r], 0, 0, 0);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        if (g == GS - D) {
+          __builtin_amdgcn_s_waitcnt(kLdsRead);
+          __builtin_amdgcn_s_barrier();
+          read_w(nst, nj, npan, 0, (P + QS) & 1);
+          read_a(nst, nj, npan, 0, (g + D) % AR);
+        }
+      }
+      cst = nst;
+    };
+    bool ff = false;
+    if constexpr (kFp8) {
+      uint32_t hit = 0;
+      for (uint32_t e = lane; e < TM * KB / 16; e += 64) {
+        const v4u v = reinterpret_cast<const v4u*>(pan + 256)[e];
+        hit |= has_ff(v.x) | has_ff(v.y) | has_ff(v.z) | has_ff(v.w);
+      }
+      if (lane < KB / 4) hit |= has_ff(reinterpret_cast<const uint32_t*>(pan)[lane]);
+      ff = __builtin_amdgcn_ballot_w64(hit != 0) != 0;
+      if (ff) bad |= kErrScale;
+    }
+    auto run = [&](auto FF) __attribute__((always_inline)) {
+      // one slice a step: two steps a trip, so that the W buffers are constant
+#pragma unroll 1
+      for (uint32_t j = 0; j < steps; j += QS % 2 ? 2 : 1) {
+        step(j, std::integral_constant<int, 0>{}, FF);
+        if constexpr (QS % 2) step(j + 1, std::integral_constant<int, 1>{}, FF);
+      }
+    };
+    if (kFp8 && ff) run(std::true_type{});
+    else run(std::false_type{});
+    const uint32_t orow = row0 + wm * MW * 16 + lr, ocol = col0 + wn * NW * 16 + 4 * lg;
+    bool nonfin = false;
+#pragma unroll
+    for (int r = 0; r < MW; ++r)
+#pragma unroll
+      for (int n = 0; n < NW; ++n) nonfin |= orow + r * 16 < p.m && !finite4(acc[n][r]);
+    if (!__builtin_amdgcn_ballot_w64(nonfin)) {
+      // 16 rows x 128 bytes at a time through the wave's own LDS, so that
+      // every store instruction writes whole 128-byte lines (8 rows)
+      uint8_t* const st = smem + ST * S::kStage + 2 * S::kPanelOne + wv * (16 * kOutPitch);
+      uint8_t* const put = st + lr * kOutPitch;
+      const uint8_t* const get = st + (lane >> 3) * kOutPitch + (lane & 7) * 16;
+      const uint32_t OSZ = p.out_f32 ? 4 : 2;
+      const uint32_t grow = row0 + wm * MW * 16 + (lane >> 3);
+      uint8_t* const gout = static_cast<uint8_t*>(p.out) +
+                            ((uint64_t)grow * p.out_row_stride + (uint64_t)prob * p.out_prob_col + col0 + wn * NW * 16) * OSZ +
+                            (lane & 7) * 16;
+      const uint64_t pitch = p.out_row_stride * OSZ;
+      auto flush = [&](int r, uint32_t at) __attribute__((always_inline)) {
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+          if (grow + r * 16 + h * 8 < p.m)
+            *reinterpret_cast<v4i*>(gout + (r * 16 + h * 8) * pitch + at) =
+                *reinterpret_cast<const v4i*>(get + h * 8 * kOutPitch);
+      };
+#pragma unroll
+      for (int r = 0; r < MW; ++r) {
+        if (p.out_f32) {
+#pragma unroll
+          for (int n = 0; n < NW; ++n) {
+            *reinterpret_cast<v4f*>(put + (n & 1) * 64 + lg * 16) = acc[n][r];
+            if (n & 1) flush(r, (n >> 1) * 128);
+          }
+        } else {
+#pragma unroll
+          for (int n = 0; n < NW; ++n)
+            *reinterpret_cast<uint2*>(put + n * 32 + lg * 8) =
+                uint2{f32x2_to_bf16x2(acc[n][r][0], acc[n][r][1]), f32x2_to_bf16x2(acc[n][r][2], acc[n][r][3])};
+          flush(r, 0);
+        }
+      }
+    } else {
+      // rare: one 16-column block at a time, its values picked by selects
+#pragma unroll 1
+      for (int b = 0; b < MW * NW * 4; ++b) {
+        float v = 0.0f;
+#pragma unroll
+        for (int r = 0; r < MW; ++r)
+#pragma unroll
+          for (int n = 0; n < NW; ++n)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v = b == (r * NW + n) * 4 + e ? acc[n][r][e] : v;
+        const uint32_t row = orow + b / (4 * NW) * 16, col = ocol + b / 4 % NW * 16 + (b & 3);
+        if (row >= p.m) continue;
+        if (__builtin_isfinite(v)) store1(p, row, prob, col, v);
+        else store_nonfinite<OP>(p, row, prob, col, v, bad);
+      }
+    }
+  }
+  if (bad) raise(p, bad);
+}
+
+template <int OP, int MB, int NB>
+void launch_tile(TileParams p, hipStream_t s) {
+  p.m_tiles = (p.m + 16 * MB - 1) / (16 * MB);
+  p.n_tiles = p.n / (16 * NB);
+  const uint32_t grid = (p.m_tiles * p.n_tiles * p.problems + 7) / 8 * 8;
+  hipLaunchKernelGGL((tile_gemm_kernel<OP, MB, NB>), dim3(grid), dim3(kThreads), 0, s, p);
+}
+
+template <int OP, int MB, int NB, int SBW>
+void launch_grid(TileParams p, uint32_t cus, hipStream_t s) {
+  p.m_tiles = (p.m + 16 * MB - 1) / (16 * MB);
+  p.n_tiles = p.n / (16 * NB);
+  const uint32_t grid = std::min((p.m_tiles * p.n_tiles * p.problems + 7) / 8 * 8, cus / 8 * 8);
+  hipLaunchKernelGGL((tile_grid_kernel<OP, MB, NB, SBW>), dim3(grid), dim3(kThreads), 0, s, p);
+}
+
+template <int OP, int MB>
+void launch_nb(int nb, const TileParams& p, hipStream_t s) {
+  switch (nb) {
+    case 1: launch_tile<OP, MB, 1>(p, s); break;
+    case 2: launch_tile<OP, MB, 2>(p, s); break;
+    case 3:
+      if constexpr (OP == kTileBf16) launch_tile<OP, MB, 3>(p, s);
+      break;
+    case 4: launch_tile<OP, MB, 4>(p, s); break;
+    case 8:
+      if constexpr (MB <= 4) launch_tile<OP, MB, 8>(p, s);
+      break;
+  }
+}
+
+template <int OP>
+void launch_pick(const TilePick& t, const TileParams& p, hipStream_t s) {
+  if (t.grid) {
+    if (t.mb == 8) launch_grid<OP, 8, 8, kGridStep>(p, kCus, s);
+    else if (t.mb == 12) launch_grid<OP, 12, 8, kGridStep>(p, kCus, s);
+    else if constexpr (OP == kTileBf16) launch_grid<OP, 16, 8, kGridStep>(p, kCus, s);
+    return;
+  }
+  switch (t.mb) {
+    case 1: launch_nb<OP, 1>(t.nb, p, s); break;
+    case 2: launch_nb<OP, 2>(t.nb, p, s); break;
+    case 3: launch_nb<OP, 3>(t.nb, p, s); break;
+    case 4: launch_nb<OP, 4>(t.nb, p, s); break;
+    case 5: launch_nb<OP, 5>(t.nb, p, s); break;
+    case 6: launch_nb<OP, 6>(t.nb, p, s); break;
+    case 8: launch_nb<OP, 8>(t.nb, p, s); break;
+  }
+}
+
+}  // namespace
+
+// The tile for a shape, by an estimate of its time: the rounds of tiles on the
+// CUs times what a CU loads for one (at the ~64 GB/s it takes in while part of
+// its lines come from HBM), no less than the weights at the 6.2 TB/s they
+// stream at, and 1.5 us for each round after the first (the start-up that the
+// tile-walking kernel hides).  16 x 16 tiles share a CU two at a time: their
+// weights were measured to stream at 7 TB/s (12288 x 4096 bf16 at m 8: 16.5
+// us, 18.4 with 16 x 48 tiles) and a round is 512 of them, 1.1 us apart.
+// Over 100 shapes (m 1-2048; Qwen3-8B, Qwen3 MLP and DeepSeek projections) the
+// choice was the fastest measured tile or within 13 % of it, 1 % on average.
+TilePick PickTile(bool bf16, uint32_t m, uint32_t n, uint32_t row_bytes, uint32_t problems) {
+  TilePick best;
+  double best_ns = 0.0;
+  const double w_bytes = (double)n * problems * row_bytes;
+  auto consider = [&](uint32_t mb, uint32_t nb, bool grid) {
+    if (n % (16 * nb) || (mb > 1 && 16 * (mb - 1) >= m && mb < 8)) return;
+    const uint64_t tiles = (uint64_t)((m + 16 * mb - 1) / (16 * mb)) * (n / (16 * nb)) * problems;
+    const bool paired = mb == 1 && nb == 1;
+    const double rounds = (double)((tiles + kCus - 1) / kCus);
+    const double load = rounds * 16.0 * (mb + nb) * row_bytes / 64.0;
+    const double hbm = w_bytes / (paired ? 7000.0 : 6200.0);
+    const double start = grid     ? 0.0
+                         : paired ? (double)((tiles + 2 * kCus - 1) / (2 * kCus) - 1) * 1100.0
+                                  : (rounds - 1.0) * 1500.0;
+    const double ns = std::max(load, hbm) + start + 0.02 * load;
+    // as good: the more nearly square tile, then the taller one
+    const bool tie = ns < best_ns + 1e-6 && (std::min(mb, nb) > std::min(best.mb, best.nb) ||
+                                             (std::min(mb, nb) == std::min(best.mb, best.nb) && mb > best.mb));
+    if (!best.mb || ns < best_ns - 1e-6 || tie) {
+      best = TilePick{mb, nb, grid};
+      best_ns = ns;
+    }
+  };
+  for (uint32_t mb : {1u, 2u, 3u, 4u, 5u, 6u, 8u})
+    for (uint32_t nb : {1u, 2u, 3u, 4u, 8u})
+      if ((bf16 || nb != 3) && (nb != 8 || mb <= 4)) consider(mb, nb, false);
+  // (a tile's scale panel is reused two tiles later: the ring must not run
+  // further ahead than one tile)
+  if (row_bytes / kGridStep >= 8) {
+    consider(8, 8, true);
+    consider(12, 8, true);
+    if (bf16) consider(16, 8, true);
+  }
+  return best;
+}
+
+bool TileGemmTakes(const TileGemmArgs& a) {
+  const uint64_t rb = a.bf16 ? 2ull * a.k : a.k, osz = a.out_kind == kOutF32 ? 4 : 2;
+  if (a.m == 0 || a.n == 0 || a.k == 0 || a.problems == 0 || rb % SB || a.n % (a.bf16 ? 16 : 128)) return false;
+  if (a.out_kind != kOutBf16 && a.out_kind != kOutF32) return false;
+  const uint64_t rows = (uint64_t)(a.m - 1) * a.a_row_stride + (uint64_t)(a.problems - 1) * a.a_prob_row + 1;
+  const uint64_t stride = a.out_row_stride ? a.out_row_stride : a.n;
+  // 32-bit byte offsets into A and within a W tile, 16-byte loads and stores
+  if (rows > a.a_rows_total || rows * rb > 0xffffffffull || 128ull * rb > 0xffffffffull) return false;
+  if ((uint64_t)a.n * a.problems / 16 * ((a.m + 15) / 16) > 0x3fffffffull) return false;
+  if ((reinterpret_cast<uintptr_t>(a.a) | reinterpret_cast<uintptr_t>(a.w) | reinterpret_cast<uintptr_t>(a.out)) % 16 ||
+      stride * osz % 16 || (uint64_t)a.out_prob_col * osz % 16)
+    return false;
+  if (a.bf16) return true;
+  return a.k % 512 == 0 && a.k / 128 <= kMaxKb &&
+         (reinterpret_cast<uintptr_t>(a.a_scale) | reinterpret_cast<uintptr_t>(a.w_scale)) % 4 == 0;
+}
+
+St LaunchTileGemm(const TileGemmArgs& a) {
+  if (!a.a || !a.w || !a.out || !a.stream || (!a.bf16 && (!a.a_scale || !a.w_scale || !a.error_flag)))
+    return Invalid("tile_gemm_null_argument");
+  if (!TileGemmTakes(a)) return Invalid("tile_gemm_shape_invalid");
+  TileParams p{};
+  p.a = static_cast<const uint8_t*>(a.a);
+  p.w = static_cast<const uint8_t*>(a.w);
+  p.a_scale = a.a_scale;
+  p.w_scale = a.w_scale;
+  p.out = a.out;
+  p.err = a.error_flag;
+  p.m = a.m;
+  p.n = a.n;
+  p.row_bytes = a.bf16 ? 2 * a.k : a.k;
+  p.problems = a.problems;
+  p.a_row_stride = a.a_row_stride;
+  p.a_prob_row = a.a_prob_row;
+  p.out_row_stride = a.out_row_stride ? a.out_row_stride : a.n;
+  p.out_prob_col = a.out_prob_col;
+  p.out_f32 = a.out_kind == kOutF32;
+  p.write_nonfinite = a.write_nonfinite;
+  p.check_codes = a.check_codes;
+  if (a.error_flag) {
+    p.err_code = a.err_code_bit;
+    p.err_scale = a.err_scale_bit;
+    p.err_nonfinite = a.err_nonfinite_bit;
+  }
+  const TilePick t = PickTile(a.bf16, a.m, a.n, p.row_bytes, a.problems);
+  St s = RequireCleanLastError();
+  if (!s.ok()) return s;
+  if (a.bf16) launch_pick<kTileBf16>(t, p, a.stream);
+  else launch_pick<kTileFp8>(t, p, a.stream);
+  return AfterLaunch("tile_gemm_launch_failed");
+}
+
+}  // namespace pih_amd

@@ -197,6 +197,38 @@ struct BigTileArgs {
   bool code_check = false;
 };
 St LaunchBigTileGemm(const BigTileArgs& a, bool* codes_in_tiles = nullptr);
+// Dense GEMM of any batch size on tiles chosen per shape (gemm_tile.hip):
+// out [m, n] = A [m, k] . W [n, k]^T, bf16 operands, or e4m3 operands with
+// UE8M0 scales (k % 512 == 0, k <= 8192), one or more strided problems as in
+// BigTileArgs.  TileGemmTakes: the shapes and alignments it runs (bf16: n %
+// 16 == 0, k % 128 == 0; operands, output and its rows on 16-byte boundaries).
+struct TileGemmArgs {
+  const void* a = nullptr;
+  const uint8_t* a_scale = nullptr;
+  const void* w = nullptr;
+  const uint8_t* w_scale = nullptr;
+  void* out = nullptr;
+  uint32_t* error_flag = nullptr;  // optional for bf16
+  hipStream_t stream = nullptr;
+  uint32_t m = 0, n = 0, k = 0;
+  uint32_t problems = 1, a_rows_total = 0, a_row_stride = 1, a_prob_row = 0;
+  uint64_t out_row_stride = 0;
+  uint32_t out_prob_col = 0;
+  bool bf16 = false;
+  OutKind out_kind = kOutBf16;
+  bool check_codes = false;  // e4m3 NaN codes count as 0 and raise err_code_bit
+  uint32_t err_code_bit = 1u, err_scale_bit = 2u, err_nonfinite_bit = 4u;
+  bool write_nonfinite = false;
+};
+bool TileGemmTakes(const TileGemmArgs& a);
+St LaunchTileGemm(const TileGemmArgs& a);
+// The tile it runs: 16 mb x 16 nb output elements, one per block or (grid)
+// one block per CU walking them
+struct TilePick {
+  uint32_t mb = 0, nb = 0;
+  bool grid = false;
+};
+TilePick PickTile(bool bf16, uint32_t m, uint32_t n, uint32_t row_bytes, uint32_t problems);
 // K splits for a dense big-tile GEMM of k_steps 128-byte K steps (1: none):
 // below a round of tiles on the 256 CUs
 uint32_t DenseKSplits(uint32_t m, uint32_t n, uint32_t k_steps);

@@ -1,0 +1,218 @@
+"""GPU parity of the per-shape tiles (gemm_tile.hip): BF16 and e4m3 (UE8M0)
+dense GEMMs at the edges of their tiles.
+
+Operands are small integers (e4m3: integers times power-of-two scales within
+a factor of 8), so every product and every partial sum is an integer multiple
+of one power of two below 2^24 of it: exact in fp32 in any order.  The fp32
+output must therefore equal the float64 product bit for bit, and the bf16
+output its rounding, whatever tile, K split or order the kernel uses."""
+import numpy as np
+import pytest
+
+from pih_amd import abi
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def eng():
+    import torch
+
+    from pih_amd.device import engine_stream
+
+    with engine_stream() as s:
+        yield s
+        torch.cuda.synchronize()
+
+
+def _ints(shape, seed, high=3):
+    import torch
+
+    g = torch.Generator(device="cuda")
+    g.manual_seed(seed)
+    return torch.randint(-high, high + 1, shape, device="cuda", generator=g).float()
+
+
+# m, n, k around: one and two rows, whole and ragged 16-row blocks, 1-5
+# blocks a tile, 48-column tiles (n / 16 not even), fewer K steps than LDS
+# stages (k 128: one step), several rounds, the tile-walking kernel (128 x
+# 128, 192 x 128 and 256 x 128 tiles, more tiles than CUs and fewer)
+BF16 = [(2, 16, 128), (3, 64, 256), (16, 1024, 384), (17, 4096, 128), (33, 48, 1152), (48, 768, 512),
+        (57, 12288, 512), (64, 1024, 4096), (65, 256, 640), (80, 4096, 256), (127, 512, 1024), (200, 12288, 512),
+        (301, 1024, 2048), (600, 9216, 512), (1000, 4096, 1024), (2048, 4096, 512), (2047, 12288, 512)]
+
+
+@pytest.mark.parametrize("m,n,k", BF16)
+def test_bf16_exact(eng, m, n, k):
+    import torch
+
+    from pih_amd.linear import bf16_gemm
+
+    a, w = _ints((m, k), m + k), _ints((n, k), n + k + 1)
+    ref = a.double() @ w.double().T
+    f32 = bf16_gemm(a.bfloat16(), w.bfloat16(), abi.OUTPUT_F32, out=torch.full((m, n), float("nan"), device="cuda"))
+    b16 = bf16_gemm(a.bfloat16(), w.bfloat16())
+    torch.cuda.synchronize()
+    assert torch.equal(f32.double(), ref)
+    assert torch.equal(b16, ref.float().bfloat16())
+
+
+@pytest.mark.parametrize("m,n,k", [(5, 64, 256), (40, 128, 384)])
+def test_bf16_unaligned_operand(eng, m, n, k):
+    """W 8 bytes off a 16-byte boundary: the GEMV the call took before."""
+    import torch
+
+    from pih_amd.linear import bf16_gemm
+
+    a, w = _ints((m, k), 1).bfloat16(), _ints((n, k), 2).bfloat16()
+    buf = torch.empty(n * k + 8, dtype=torch.bfloat16, device="cuda")
+    off = buf[4:4 + n * k].view(n, k)
+    off.copy_(w)
+    got = bf16_gemm(a, off, abi.OUTPUT_F32)
+    torch.cuda.synchronize()
+    assert off.data_ptr() % 16 == 8 and torch.equal(got.double(), a.double() @ w.double().T)
+
+
+def _fp8(m, n, k, seed):
+    """e4m3 codes of integers in [-3, 3] and scale bytes 126..128, with the
+    float64 operands they stand for."""
+    import torch
+
+    a, w = _ints((m, k), seed), _ints((n, k), seed + 1)
+    sa = 127 + _ints((m, k // 128), seed + 2, 1).to(torch.uint8)
+    sw = 127 + _ints((n // 128, k // 128), seed + 3, 1).to(torch.uint8)
+    code = lambda v: v.to(torch.float8_e4m3fn).view(torch.uint8).clone()  # noqa: E731
+    return code(a), sa, code(w), sw
+
+
+def _expect(a, sa, w, sw):
+    """(float64 product with NaN codes and 0xFF-scaled blocks as 0)"""
+    import torch
+
+    m, k = a.shape
+    n = w.shape[0]
+
+    def val(c):
+        v = c.view(torch.float8_e4m3fn).double()
+        return torch.where(torch.isnan(v), torch.zeros_like(v), v)
+
+    def scale(s):
+        return torch.where(s == 255, torch.zeros_like(s, dtype=torch.float64), torch.exp2(s.double() - 127))
+
+    av = (val(a).view(m, k // 128, 128) * scale(sa)[:, :, None]).view(m, k)
+    wv = (val(w).view(n // 128, 128, k // 128, 128) * scale(sw)[:, None, :, None]).view(n, k)
+    return av @ wv.T
+
+
+def _run_fp8(a, sa, w, sw, out_type):
+    import torch
+
+    from pih_amd.device import ptr, stream_handle
+
+    m, k = a.shape
+    n = w.shape[0]
+    out = torch.full((m, n), float("nan"), device="cuda", dtype=torch.float32 if out_type == 2 else torch.bfloat16)
+    flag = torch.zeros(1, dtype=torch.int32, device="cuda")
+    r = abi.request(abi.DS["fp8_gemm"], activation_e4m3=ptr(a), activation_scale_bits=ptr(sa), weight_e4m3=ptr(w),
+                    weight_scale_bits=ptr(sw), output=ptr(out), error_flag=ptr(flag), stream=stream_handle(), m=m, n=n,
+                    k=k, output_type=out_type)
+    st = abi.deepseek_pack().call("launch_fp8_gemm", r)
+    assert st.code == abi.OK, st
+    torch.cuda.synchronize()
+    return out, int(flag.item())
+
+
+# k 8192 is the deepest scale panel; k 512 and 1024 have fewer steps than
+# stages; 768 (not a multiple of 512) and 8704 (deeper) stay on other kernels
+FP8 = [(1, 128, 512), (3, 1024, 1024), (4, 4096, 8192), (16, 2048, 512), (17, 128, 1536), (40, 256, 768),
+       (50, 4096, 512), (75, 1024, 2048), (129, 4096, 1024), (33, 128, 8704), (301, 2048, 1024), (301, 32768, 1024),
+       (700, 4096, 2048), (2048, 1024, 1024), (2047, 8192, 1024)]
+
+
+@pytest.mark.parametrize("m,n,k", FP8)
+def test_fp8_exact(eng, m, n, k):
+    import torch
+
+    a, sa, w, sw = _fp8(m, n, k, 7 * m + n + k)
+    ref = _expect(a, sa, w, sw)
+    for out_type in (1, 2):
+        got, flag = _run_fp8(a, sa, w, sw, out_type)
+        assert flag == 0
+        assert torch.equal(got, ref.float().bfloat16() if out_type == 1 else ref.float())
+
+
+@pytest.mark.parametrize("m,n,k", [(20, 256, 1024), (301, 2048, 1024), (700, 8192, 1024)])
+def test_fp8_codes_and_invalid_scales(eng, m, n, k):
+    """NaN codes count as 0 and raise bit 1, 0xFF scales leave their block out
+    and raise bit 2, in one-tile-per-block and in walked tiles; a code in a
+    block that a 0xFF scale leaves out raises bit 2 alone."""
+    import torch
+
+    a, sa, w, sw = _fp8(m, n, k, m)
+    a[m - 1, 5], w[n - 1, k - 1] = 0x7F, 0xFF
+    got, flag = _run_fp8(a, sa, w, sw, 2)
+    assert flag == 1 and torch.equal(got, _expect(a, sa, w, sw).float())
+    a, sa, w, sw = _fp8(m, n, k, m)
+    sa[m // 2, 3], sw[n // 128 - 1, 1] = 255, 255
+    got, flag = _run_fp8(a, sa, w, sw, 2)
+    assert flag == 2 and torch.equal(got, _expect(a, sa, w, sw).float())
+    a[m // 2, 3 * 128 + 7] = 0x7F
+    got, flag = _run_fp8(a, sa, w, sw, 2)
+    assert flag & 2 and torch.equal(got, _expect(a, sa, w, sw).float())
+
+
+@pytest.mark.parametrize("t", [1, 7, 65, 130])
+def test_grouped_fp8_exact(eng, t):
+    """Strided problems (4 groups of 256 x 512 over interleaved rows): the
+    quantised rows' own codes and scales give the expected product; fp32 sums
+    of codes up to 448 are not exact, so 512 terms' rounding bounds the error
+    (512 x 2^-24 of the sum of magnitudes) beside bf16's half ulp."""
+    import torch
+
+    from pih_amd.device import ptr, stream_handle
+
+    g, n, k = 4, 256, 512
+    x = _ints((t * g, k), t, 100).bfloat16()
+    _, _, w, sw = _fp8(1, g * n, k, t)
+    aq = torch.empty(t * g, k, dtype=torch.uint8, device="cuda")
+    sa = torch.empty(t * g, k // 128, dtype=torch.uint8, device="cuda")
+    out = torch.full((t, g * n), float("nan"), dtype=torch.bfloat16, device="cuda")
+    flag = torch.zeros(1, dtype=torch.int32, device="cuda")
+    r = abi.request(abi.DS["grouped_fp8_gemm"], input_bf16=ptr(x), activation_e4m3=ptr(aq),
+                    activation_scale_bits=ptr(sa), weight_e4m3=ptr(w), weight_scale_bits=ptr(sw), output_bf16=ptr(out),
+                    error_flag_u32=ptr(flag), stream=stream_handle(), token_count=t, group_count=g,
+                    output_per_group=n, input_per_group=k)
+    st = abi.deepseek_pack().call("launch_grouped_fp8_gemm", r)
+    assert st.code == abi.OK, st
+    torch.cuda.synchronize()
+    assert int(flag.item()) == 0
+    av = (aq.view(torch.float8_e4m3fn).double().view(t, g, k // 128, 128) *
+          torch.exp2(sa.double() - 127).view(t, g, k // 128, 1)).view(t, g, k)
+    wv = (w.view(torch.float8_e4m3fn).double().view(g, n // 128, 128, k // 128, 128) *
+          torch.exp2(sw.double() - 127).view(g, n // 128, 1, k // 128, 1)).view(g, n, k)
+    for q in range(g):
+        ref = av[:, q] @ wv[q].T
+        mag = av[:, q].abs() @ wv[q].abs().T
+        err = (out[:, q * n:(q + 1) * n].double() - ref).abs()
+        assert bool((err <= ref.abs() * 2.0 ** -8 + mag * k * 2.0 ** -24).all())
+
+
+def test_lm_head_nonfinite_bits_many_rows(eng):
+    """Above 128 rows the DeepSeek head runs on the per-shape tiles: a
+    non-finite logit is stored and raises 128, the element behind it 64."""
+    import torch
+
+    from pih_amd.device import flag_value
+    from pih_amd.linear import deepseek_lm_head
+
+    x, w = _ints((150, 4096), 3).bfloat16(), _ints((129280, 4096), 4).bfloat16()
+    out, flag = deepseek_lm_head(x, w)
+    torch.cuda.synchronize()
+    ref = torch.cat([(x.double() @ v.double().T).float() for v in w.split(16160)], dim=1)
+    assert flag_value(flag) == 0 and torch.equal(out, ref)
+    w[70000, 9] = float("inf")
+    out, flag = deepseek_lm_head(x, w)
+    torch.cuda.synchronize()
+    assert flag_value(flag) == 128 | 64
+    keep = np.arange(129280) != 70000
+    assert torch.equal(out[:, keep], ref[:, keep]) and not bool(torch.isfinite(out[:, 70000]).any())
