@@ -1133,6 +1133,9 @@ St LaunchW4a16(const W4a16Args& a) {
     return Invalid("w4a16_shape_invalid");
   St clean = RequireCleanLastError();
   if (!clean.ok()) return clean;
+  bool taken;
+  const St tile = LaunchW4a16Tile(&a, 1, taken);
+  if (!tile.ok() || taken) return tile;
   GemvParams p{};
   p.x = a.x;
   p.w = a.qweight;
@@ -1176,7 +1179,8 @@ St LaunchW4a16Grouped(const W4a16Args* probs, uint32_t count) {
   St clean = RequireCleanLastError();
   if (!clean.ok()) return clean;
   bool taken;
-  St st;
+  St st = LaunchW4a16Tile(probs, count, taken);
+  if (!st.ok() || taken) return st;
   if (a0.m <= kSmallM)
     st = a0.symmetric ? launch_group_lds<kWSym>(g, a0.stream, taken) : launch_group_lds<kWAsym>(g, a0.stream, taken);
   else

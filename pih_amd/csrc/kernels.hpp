@@ -286,6 +286,9 @@ St LaunchW4a16(const W4a16Args& a);
 // up to 8 problems with one m, k and format in one launch (x, qweight,
 // scales, zeros, out and n per problem; the rest from probs[0])
 St LaunchW4a16Grouped(const W4a16Args* probs, uint32_t count);
+// batches of 2-32 rows on tiles (w4a16_tile.hip), after the callers' checks;
+// `taken` false when the GEMV kernels are the faster or only ones
+St LaunchW4a16Tile(const W4a16Args* probs, uint32_t count, bool& taken);
 uint64_t W4a16WorkspaceBytes(uint32_t m, uint32_t n, uint32_t k);
 // exact dequant (q - z) * s (or q * s) to fp32 [n, k]
 St LaunchW4a16Dequant(const W4a16Args& a, float* out);
