@@ -375,9 +375,11 @@ _loaded: Dict[str, KernelPack] = {}
 def load_pack(path: str, contract: str, expected_sha256: Optional[str] = None) -> KernelPack:
     """Load a Kernel Pack with the reference loader's checks; packs are never
     unloaded (kernel_pack_loader.cpp:117-119)."""
-    path = os.path.abspath(path)
-    if path in _loaded:
-        pack = _loaded[path]
+    pack = _loaded.get(path)
+    if pack is None:
+        path = os.path.abspath(path)
+        pack = _loaded.get(path)
+    if pack is not None:
         if pack.pack_abi != contract:
             raise PackError(f"contract mismatch: pack exports {pack.pack_abi!r}, caller wants {contract!r}")
         return pack

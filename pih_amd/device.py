@@ -23,21 +23,45 @@ def require_gpu() -> None:
 
 def stream() -> "torch.cuda.Stream":
     global _stream
-    require_gpu()
     if _stream is None:
+        require_gpu()
         _stream = torch.cuda.Stream()
     return _stream
 
 
-@contextlib.contextmanager
-def engine_stream():
-    s = stream()
-    with torch.cuda.stream(s):
-        yield s
+class engine_stream(contextlib.ContextDecorator):
+    """``with engine_stream() as s``: the engine stream is torch's current
+    stream inside.  The same switch as ``torch.cuda.stream(s)``; entering and
+    leaving through the two calls that one ends in took 7.6 -> 1.6 us, of the
+    ~27 us of host time around a four-launch decode block."""
+
+    def _recreate_cm(self):  # as a decorator: a context of its own per call
+        return engine_stream()
+
+    def __enter__(self):
+        s = stream()
+        self._other = None
+        if torch._C._cuda_getDevice() != s.device_index:
+            # another device is current: torch's own context restores both
+            self._other = torch.cuda.stream(s)
+            self._other.__enter__()
+        else:
+            self._previous = torch._C._cuda_getCurrentStream(s.device_index)
+            torch._C._cuda_setStream(stream_id=s.stream_id, device_index=s.device_index, device_type=s.device_type)
+        return s
+
+    def __exit__(self, *exc):
+        if self._other is not None:
+            self._other.__exit__(*exc)
+        else:
+            sid, index, kind = self._previous
+            torch._C._cuda_setStream(stream_id=sid, device_index=index, device_type=kind)
+        return False
 
 
 def stream_handle() -> int:
-    h = torch.cuda.current_stream().cuda_stream
+    # the current stream's handle without a Stream object (2.8 -> 0.3 us)
+    h = torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
     if h == 0:
         raise RuntimeError("pih_amd: launches need an explicit stream; run under pih_amd.device.engine_stream()")
     return h
