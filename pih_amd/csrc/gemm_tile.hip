@@ -32,7 +32,9 @@
 // them (plugins/kernels/deepseek-v4-sm89/native/deepseek_fp8_gemm.cu:11-70):
 // a code turns every sum over its row into a NaN, so an element that came out
 // non-finite looks for codes in its two operand rows and, finding one, is
-// summed again the reference's way.  A 0xFF scale's block adds nothing.
+// summed again the reference's way.  A 0xFF scale's block adds nothing, also
+// where the caller asked for no code check (the grouped GEMM): the sum from
+// before the block's MFMA is kept, so its codes are never seen.
 #include <algorithm>
 #include <type_traits>
 
@@ -159,6 +161,17 @@ __device__ __forceinline__ void raise(const TileParams& p, uint32_t bad) {
   if (bits) atomicOr(p.err, bits);
 }
 
+// A block under a 0xFF scale adds nothing, whatever its codes: a lane's four
+// results belong to one A row (scale byte as) and one 128-row W block (ws),
+// and the sum before the MFMA is kept.  (Zeroed operands or a scale of 0
+// would do for finite values only: a NaN code in the other operand, or in
+// the skipped one, stays a NaN.)
+__device__ __forceinline__ v4f without_ff_block(uint32_t ws, uint32_t as, v4f before, v4f after) {
+  const bool skip = ws == 0xffu || as == 0xffu;
+  return v4f{skip ? before[0] : after[0], skip ? before[1] : after[1], skip ? before[2] : after[2],
+             skip ? before[3] : after[3]};
+}
+
 __device__ __forceinline__ uint32_t has_ff(uint32_t v) { return (~v - 0x01010101u) & v & 0x80808080u; }
 
 template <int OP, int MB, int NB>
@@ -281,30 +294,20 @@ __global__ __launch_bounds__(kThreads, 1) void tile_gemm_kernel(TileParams p) {
         return v8i{x[0], x[1], x[2], x[3], y[0], y[1], y[2], y[3]};
       };
       const uint32_t kb = 2 * j + kh;
-      uint32_t ws = pw[kb];
-      const bool wff = decltype(FF)::value && ws == 0xffu;
-      if (wff) ws = 0;
+      const uint32_t ws = pw[kb];
       v8i wf[NW];
 #pragma unroll
       for (int n = 0; n < NW; ++n) wf[n] = frag(sw + n * 4096);
 #pragma unroll
       for (int r = 0; r < MW; ++r) {
-        v8i af = frag(sa + r * 4096);
-        uint32_t as = pa[(mb0 * 16 + r * 16 + lr) * KB + kb];
-        if constexpr (decltype(FF)::value) {
-          // a 0xFF scale's block adds nothing: an A row's fragment becomes 0;
-          // a W block runs with both scales 0 (2^-254 times a sum below 2^25
-          // is below the fp32 range)
-          const int keep = as == 0xffu ? 0 : -1;
+        const v8i af = frag(sa + r * 4096);
+        const uint32_t as = pa[(mb0 * 16 + r * 16 + lr) * KB + kb];
 #pragma unroll
-          for (int q = 0; q < 8; ++q) af[q] &= keep;
-          as = as == 0xffu ? 127u : as;
-          as = wff ? 0u : as;
+        for (int n = 0; n < NW; ++n) {
+          const v4f sum = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(wf[n], af, acc[n][r], 0, 0, 0, (int)ws, 0,
+                                                                           (int)as);
+          acc[n][r] = decltype(FF)::value ? without_ff_block(ws, as, acc[n][r], sum) : sum;
         }
-#pragma unroll
-        for (int n = 0; n < NW; ++n)
-          acc[n][r] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(wf[n], af, acc[n][r], 0, 0, 0, (int)ws, 0,
-                                                                       (int)as);
       }
     }
   };
@@ -603,25 +606,18 @@ __global__ __launch_bounds__(kThreads, 1) void tile_grid_kernel(TileParams p) {
           else read_a(nst, nj, npan, g + D - GS, (g + D) % AR);
           if (q + 1 < QS && r == MW - D) read_w(cst, j, pan, q + 1, wb ^ 1);
         }
-        Frag a = af[g % AR];
-        uint32_t sa = as[g % AR], sw = ws[wb];
-        if constexpr (kFp8 && decltype(FF)::value) {
-          // a 0xFF scale's block adds nothing (see compute above)
-          const int keep = sa == 0xffu ? 0 : -1;
-#pragma unroll
-          for (int e = 0; e < 8; ++e) a[e] &= keep;
-          const bool wff = sw == 0xffu;
-          sa = wff ? 0u : sa == 0xffu ? 127u : sa;
-          sw = wff ? 0u : sw;
-        }
+        const Frag a = af[g % AR];
+        const uint32_t sa = as[g % AR], sw = ws[wb];
 #pragma unroll
         for (int n = 0; n < NW; ++n) {
-          if constexpr (kFp8)
-            acc[n][r] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(wf[wb][n], a, acc[n][r], 0, 0, 0, (int)sw, 0,
-                                                                         (int)sa);
-          else
+          if constexpr (kFp8) {
+            const v4f sum = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(wf[wb][n], a, acc[n][r], 0, 0, 0, (int)sw,
+                                                                             0, (int)sa);
+            acc[n][r] = decltype(FF)::value ? without_ff_block(sw, sa, acc[n][r], sum) : sum;
+          } else {
             acc[n][r] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8bf, wf[wb][n]),
                                                                 __builtin_bit_cast(v8bf, a), acc[n][r], 0, 0, 0);
+          }
         }
         __builtin_amdgcn_sched_barrier(0);
         if (g == GS - D) {

@@ -85,23 +85,30 @@ def _fp8(m, n, k, seed):
     return code(a), sa, code(w), sw
 
 
-def _expect(a, sa, w, sw):
-    """(float64 product with NaN codes and 0xFF-scaled blocks as 0)"""
+def _values(c):
     import torch
 
-    m, k = a.shape
-    n = w.shape[0]
+    v = c.view(torch.float8_e4m3fn).double()
+    return torch.where(torch.isnan(v), torch.zeros_like(v), v)
 
-    def val(c):
-        v = c.view(torch.float8_e4m3fn).double()
-        return torch.where(torch.isnan(v), torch.zeros_like(v), v)
 
-    def scale(s):
-        return torch.where(s == 255, torch.zeros_like(s, dtype=torch.float64), torch.exp2(s.double() - 127))
+def _scales(s):
+    import torch
 
-    av = (val(a).view(m, k // 128, 128) * scale(sa)[:, :, None]).view(m, k)
-    wv = (val(w).view(n // 128, 128, k // 128, 128) * scale(sw)[:, None, :, None]).view(n, k)
+    return torch.where(s == 255, torch.zeros_like(s, dtype=torch.float64), torch.exp2(s.double() - 127))
+
+
+def _product(av, w, sw):
+    """av (float64 rows) times W, its NaN codes and 0xFF-scaled blocks as 0"""
+    n, k = w.shape
+    wv = (_values(w).view(n // 128, 128, k // 128, 128) * _scales(sw)[:, None, :, None]).view(n, k)
     return av @ wv.T
+
+
+def _expect(a, sa, w, sw):
+    """(float64 product with NaN codes and 0xFF-scaled blocks as 0)"""
+    m, k = a.shape
+    return _product((_values(a).view(m, k // 128, 128) * _scales(sa)[:, :, None]).view(m, k), w, sw)
 
 
 def _run_fp8(a, sa, w, sw, out_type):
@@ -157,23 +164,23 @@ def test_fp8_codes_and_invalid_scales(eng, m, n, k):
     got, flag = _run_fp8(a, sa, w, sw, 2)
     assert flag == 2 and torch.equal(got, _expect(a, sa, w, sw).float())
     a[m // 2, 3 * 128 + 7] = 0x7F
+    w[n - 1, 128 + 9] = 0xFF
     got, flag = _run_fp8(a, sa, w, sw, 2)
-    assert flag & 2 and torch.equal(got, _expect(a, sa, w, sw).float())
+    assert flag == 2 and torch.equal(got, _expect(a, sa, w, sw).float())
+    # a W code that the row's 0xFF scale leaves out, but no other row's
+    w[5, 3 * 128 + 1] = 0x7F
+    got, flag = _run_fp8(a, sa, w, sw, 2)
+    assert flag == 3 and torch.equal(got, _expect(a, sa, w, sw).float())
 
 
-@pytest.mark.parametrize("t", [1, 7, 65, 130])
-def test_grouped_fp8_exact(eng, t):
-    """Strided problems (4 groups of 256 x 512 over interleaved rows): the
-    quantised rows' own codes and scales give the expected product; fp32 sums
-    of codes up to 448 are not exact, so 512 terms' rounding bounds the error
-    (512 x 2^-24 of the sum of magnitudes) beside bf16's half ulp."""
+def _run_grouped(t, g, n, k, w, sw, seed):
+    """launch_grouped_fp8_gemm on integer rows: (output, flag, the float64
+    activations [t, g, k] its quantised rows stand for)."""
     import torch
 
     from pih_amd.device import ptr, stream_handle
 
-    g, n, k = 4, 256, 512
-    x = _ints((t * g, k), t, 100).bfloat16()
-    _, _, w, sw = _fp8(1, g * n, k, t)
+    x = _ints((t * g, k), seed, 100).bfloat16()
     aq = torch.empty(t * g, k, dtype=torch.uint8, device="cuda")
     sa = torch.empty(t * g, k // 128, dtype=torch.uint8, device="cuda")
     out = torch.full((t, g * n), float("nan"), dtype=torch.bfloat16, device="cuda")
@@ -185,16 +192,48 @@ def test_grouped_fp8_exact(eng, t):
     st = abi.deepseek_pack().call("launch_grouped_fp8_gemm", r)
     assert st.code == abi.OK, st
     torch.cuda.synchronize()
-    assert int(flag.item()) == 0
     av = (aq.view(torch.float8_e4m3fn).double().view(t, g, k // 128, 128) *
           torch.exp2(sa.double() - 127).view(t, g, k // 128, 1)).view(t, g, k)
-    wv = (w.view(torch.float8_e4m3fn).double().view(g, n // 128, 128, k // 128, 128) *
-          torch.exp2(sw.double() - 127).view(g, n // 128, 1, k // 128, 1)).view(g, n, k)
+    return out, int(flag.item()), av
+
+
+def _check_grouped(out, av, w, sw, g, n):
+    """fp32 sums of codes up to 448 are not exact, so k terms' rounding bounds
+    the error (k x 2^-24 of the sum of magnitudes) beside bf16's half ulp."""
+    k = w.shape[1]
     for q in range(g):
-        ref = av[:, q] @ wv[q].T
-        mag = av[:, q].abs() @ wv[q].abs().T
+        wq, sq = w[q * n:(q + 1) * n], sw[q * n // 128:(q + 1) * n // 128]
+        ref = _product(av[:, q], wq, sq)
+        mag = _product(av[:, q].abs(), wq & 0x7F, sq)
         err = (out[:, q * n:(q + 1) * n].double() - ref).abs()
         assert bool((err <= ref.abs() * 2.0 ** -8 + mag * k * 2.0 ** -24).all())
+
+
+@pytest.mark.parametrize("t", [1, 7, 65, 130])
+def test_grouped_fp8_exact(eng, t):
+    """Strided problems: 4 groups of 256 x 512 over interleaved rows."""
+    g, n, k = 4, 256, 512
+    _, _, w, sw = _fp8(1, g * n, k, t)
+    out, flag, av = _run_grouped(t, g, n, k, w, sw, t)
+    assert flag == 0
+    _check_grouped(out, av, w, sw, g, n)
+
+
+# one-tile-per-block tiles (16 x 16 and 48 x 64) and walked tiles (192 x 128)
+@pytest.mark.parametrize("t,n,k", [(1, 256, 512), (7, 256, 512), (65, 2048, 1024), (700, 2048, 1024)])
+def test_grouped_fp8_codes_under_an_invalid_scale(eng, t, n, k):
+    """The grouped entry checks no codes; a W block under a 0xFF scale is left
+    out unseen all the same, NaN codes included: bit 1024 alone, and every
+    column finite."""
+    g = 4
+    _, _, w, sw = _fp8(1, g * n, k, t)
+    sw[1, 2] = 255  # W rows 128..255 of group 0, k 256..383
+    w[130, 256], w[255, 383] = 0x7F, 0xFF
+    sw[-1, 0] = 255
+    w[-1, 0:128] = 0xFF
+    out, flag, av = _run_grouped(t, g, n, k, w, sw, t)
+    assert flag == 1024
+    _check_grouped(out, av, w, sw, g, n)
 
 
 def test_lm_head_nonfinite_bits_many_rows(eng):
