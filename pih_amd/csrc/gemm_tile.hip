@@ -83,39 +83,50 @@ __device__ __forceinline__ const uint8_t* uniform_ptr(const uint8_t* p) {
 constexpr int vmcnt_at_most(int n) { return ((n >> 4) << 14) | 0x0F70 | (n & 15); }
 constexpr int kLdsRead = 0xC07F;
 
-// Output element (A row ar, column col of problem prob) the reference's way:
-// per 128-k block an fp32 sum of decoded e4m3 products in k order with NaN
-// codes as 0, a block with a 0xFF scale skipped before it is read.  False
-// when neither operand row holds a code.  (Loops kept rolled: this is rare,
-// and code in the way of the common path costs instruction fetches.)
+// Output element (A row ar, column col of problem prob) the reference's way,
+// by a whole wave (every lane the same element): per 128-k block an fp32 sum
+// of decoded e4m3 products in k order with NaN codes as 0, the blocks added
+// in order, a block with a 0xFF scale skipped before it is read.  Lane b
+// takes block b (a product of two codes is exact in fp32, so the FMA rounds
+// as the reference's multiply and add).  False when neither operand row holds
+// a code.  A call with one code in an A row or a W row (alone on the stream,
+// us, A / W; clean 6-9): 4096 -> 1024 at M 16 16.8 / 16.1, 8192 -> 4096 at M 4
+// 24 / 15, 2048 -> 4096 at M 64 23 / 22; with a lane per element, walking all
+// of K alone, 2627 / 591, 5330 / 1051 and 1324 / 513.
 __device__ __forceinline__ bool code_element(const TileParams& p, uint64_t ar, uint32_t prob, uint32_t col, float& sum,
                                              uint32_t& bits) {
-  const uint32_t RB = p.row_bytes, KB = RB / 128;
-  const uint8_t* ap = p.a + ar * RB;
-  const uint8_t* wp = p.w + ((uint64_t)prob * p.n + col) * RB;
-  const uint8_t* asp = p.a_scale + ar * KB;
-  const uint8_t* wsp = p.w_scale + ((uint64_t)prob * (p.n / 128) + col / 128) * KB;
-  uint32_t any = 0;
-  sum = 0.0f;
-  bits = 0;
+  const uint32_t RB = p.row_bytes, KB = RB / 128, lane = threadIdx.x & 63, b = min(lane, KB - 1);
+  const v4i* const ap = reinterpret_cast<const v4i*>(p.a + ar * RB) + b * 8;
+  const v4i* const wp = reinterpret_cast<const v4i*>(p.w + ((uint64_t)prob * p.n + col) * RB) + b * 8;
+  const uint32_t as = p.a_scale[ar * KB + b], ws = p.w_scale[((uint64_t)prob * (p.n / 128) + col / 128) * KB + b];
+  const bool live = lane < KB, skip = as == 0xffu || ws == 0xffu;
+  uint32_t nan = 0;
+  float local = 0.0f;
 #pragma unroll 1
-  for (uint32_t b = 0; b < KB; ++b) {
-    const bool skip = asp[b] == 0xffu || wsp[b] == 0xffu;
-    if (skip) bits |= kErrScale;
-    float local = 0.0f;
-#pragma unroll 1
-    for (uint32_t c = b * 128; c < b * 128 + 128; c += 4) {
-      const uint32_t x = *reinterpret_cast<const uint32_t*>(ap + c), y = *reinterpret_cast<const uint32_t*>(wp + c);
-      const uint32_t nx = e4m3_nan_bytes(x), ny = e4m3_nan_bytes(y);
-      any |= nx | ny;
-      if ((nx | ny) && !skip) bits |= kErrCode;
-      const uint32_t xa = e4m3_nan_to_zero(x, nx), xw = e4m3_nan_to_zero(y, ny);
-#pragma unroll 1
-      for (uint32_t e = 0; e < 32; e += 8) local = local + e4m3_decode((xa >> e) & 0xffu) * e4m3_decode((xw >> e) & 0xffu);
+  for (int c = 0; c < 8; ++c) {
+    const v4i x = ap[c], y = wp[c];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const uint32_t nx = e4m3_nan_bytes((uint32_t)x[q]), ny = e4m3_nan_bytes((uint32_t)y[q]);
+      nan |= nx | ny;
+      const int xa = (int)e4m3_nan_to_zero((uint32_t)x[q], nx), xw = (int)e4m3_nan_to_zero((uint32_t)y[q], ny);
+      const v2f a0 = __builtin_amdgcn_cvt_pk_f32_fp8(xa, false), a1 = __builtin_amdgcn_cvt_pk_f32_fp8(xa, true);
+      const v2f w0 = __builtin_amdgcn_cvt_pk_f32_fp8(xw, false), w1 = __builtin_amdgcn_cvt_pk_f32_fp8(xw, true);
+      local = __builtin_fmaf(a0[0], w0[0], local);
+      local = __builtin_fmaf(a0[1], w0[1], local);
+      local = __builtin_fmaf(a1[0], w1[0], local);
+      local = __builtin_fmaf(a1[1], w1[1], local);
     }
-    if (!skip) sum = sum + local * ue8m0_value(asp[b]) * ue8m0_value(wsp[b]);
   }
-  return any != 0;
+  const int part = __builtin_bit_cast(int, local * ue8m0_value(as) * ue8m0_value(ws));
+  const uint64_t add = __builtin_amdgcn_ballot_w64(live && !skip);
+  sum = 0.0f;
+#pragma unroll 1
+  for (uint32_t i = 0; i < KB; ++i)
+    if ((add >> i) & 1) sum = sum + __builtin_bit_cast(float, __builtin_amdgcn_readlane(part, i));
+  bits = __builtin_amdgcn_ballot_w64(live && skip) ? kErrScale : 0u;
+  if (__builtin_amdgcn_ballot_w64(live && !skip && nan)) bits |= kErrCode;
+  return __builtin_amdgcn_ballot_w64(live && nan) != 0;
 }
 
 __device__ __forceinline__ bool finite4(v4f v) {
@@ -136,29 +147,34 @@ __device__ __forceinline__ void store1(const TileParams& p, uint32_t row, uint32
   else static_cast<uint16_t*>(p.out)[o] = (uint16_t)f32_to_bf16_bits(v);
 }
 
-// The non-finite element v at (row, col): e4m3 operands that hold a NaN code
-// get the reference's sum and its bits; otherwise the value stays and raises
-// the non-finite bit, stored unless the caller leaves such elements out.
-template <int OP>
-__device__ __forceinline__ void store_nonfinite(const TileParams& p, uint32_t row, uint32_t prob, uint32_t col, float v,
+// Element v at (row, col) after the look for codes; a non-finite one raises
+// its bit and is stored unless the caller leaves such elements out.
+__device__ __forceinline__ void store_looked_at(const TileParams& p, uint32_t row, uint32_t prob, uint32_t col, float v,
                                                 uint32_t& bad) {
-  if (OP == kTileFp8 && p.check_codes) {
-    float sum;
-    uint32_t bits;
-    if (code_element(p, (uint64_t)row * p.a_row_stride + (uint64_t)prob * p.a_prob_row, prob, col, sum, bits)) {
-      v = sum;
-      bad |= bits;
-    }
-  }
   const bool fin = __builtin_isfinite(v);
   if (!fin) bad |= kErrNonFinite;
   if (fin || !p.err_nonfinite || p.write_nonfinite) store1(p, row, prob, col, v);
 }
 
+// The non-finite element v at (row, col), by a whole wave, its lane `by`
+// storing: e4m3 operands that hold a NaN code get the reference's sum and its
+// bits.
+__device__ __forceinline__ void store_nonfinite(const TileParams& p, uint32_t row, uint32_t prob, uint32_t col, float v,
+                                                uint32_t by, uint32_t& bad) {
+  float sum;
+  uint32_t bits;
+  const bool code = code_element(p, (uint64_t)row * p.a_row_stride + (uint64_t)prob * p.a_prob_row, prob, col, sum, bits);
+  if ((threadIdx.x & 63) != by) return;
+  if (code) bad |= bits;
+  store_looked_at(p, row, prob, col, code ? sum : v, bad);
+}
+
 __device__ __forceinline__ void raise(const TileParams& p, uint32_t bad) {
   const uint32_t bits = ((bad & kErrCode) ? p.err_code : 0u) | ((bad & kErrScale) ? p.err_scale : 0u) |
                         ((bad & kErrNonFinite) ? p.err_nonfinite : 0u);
-  if (bits) atomicOr(p.err, bits);
+  // (the waves of a whole output may have the same to say: only one that
+  // finds it unsaid adds to the queue at the flag)
+  if (bits & ~__hip_atomic_load(p.err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicOr(p.err, bits);
 }
 
 // A block under a 0xFF scale adds nothing, whatever its codes: a lane's four
@@ -387,8 +403,16 @@ __global__ __launch_bounds__(kThreads, 1) void tile_gemm_kernel(TileParams p) {
     else multiply_loop(std::false_type{});
   }
 
-  // ---- the waves' sums, then whole rows
+  // ---- the waves' sums, then whole rows.  Under the code check an element
+  // that came out non-finite is only marked (bit row TN + column of a map
+  // where the scale panels were), and the eight waves then share them out.
+  const bool look = kFp8 && p.check_codes;
+  uint32_t* const map = reinterpret_cast<uint32_t*>(smem + S::kRing);  // [0]: any
+  constexpr uint32_t kMapWords = TM * TN / 32;
+  static_assert(!kFp8 || (kMapWords + 1) * 4 <= S::kPanel, "the map fits the panels");
   __syncthreads();
+  if (look)
+    for (uint32_t i = tid; i <= kMapWords; i += kThreads) map[i] = 0;
   const uint32_t part = kFp8 ? kh : wv;
 #pragma unroll
   for (int n = 0; n < NW && !loader && !(kOnePair && half); ++n)
@@ -398,22 +422,57 @@ __global__ __launch_bounds__(kThreads, 1) void tile_gemm_kernel(TileParams p) {
           acc[n][r];
   __syncthreads();
   constexpr uint32_t QR = TN / 4;  // 4-column groups per row
-#pragma unroll 1
-  for (uint32_t it = tid; it < TM * QR; it += kThreads) {
-    const uint32_t row = it / QR, cq = it % QR;
-    if (row0 + row >= p.m) continue;
+  // columns 4 cq .. + 3 of a row, summed over the waves
+  auto sum4 = [&](uint32_t row, uint32_t cq) __attribute__((always_inline)) -> v4f {
     const uint8_t* s = smem + ((row >> 4) * NB + (cq >> 2)) * kSumBlock + (cq & 3) * kSumGroup + (row & 15) * 16;
     v4f v = *reinterpret_cast<const v4f*>(s);
 #pragma unroll
     for (int q = 1; q < S::kParts; ++q) v += *reinterpret_cast<const v4f*>(s + q * MB * NB * kSumBlock);
+    return v;
+  };
+  auto pick4 = [](v4f v, uint32_t i) __attribute__((always_inline)) -> float {
+    return i == 0 ? v[0] : i == 1 ? v[1] : i == 2 ? v[2] : v[3];
+  };
+#pragma unroll 1
+  for (uint32_t it = tid; it < TM * QR; it += kThreads) {
+    const uint32_t row = it / QR, cq = it % QR;
+    if (row0 + row >= p.m) continue;
+    const v4f v = sum4(row, cq);
     if (finite4(v)) {
       store4(p, row0 + row, prob, col0 + cq * 4, v);
     } else {
 #pragma unroll 1
-      for (int i = 0; i < 4; ++i) {
-        const float e = i == 0 ? v[0] : i == 1 ? v[1] : i == 2 ? v[2] : v[3];
-        if (__builtin_isfinite(e)) store1(p, row0 + row, prob, col0 + cq * 4 + i, e);
-        else store_nonfinite<OP>(p, row0 + row, prob, col0 + cq * 4 + i, e, bad);
+      for (uint32_t i = 0; i < 4; ++i) {
+        const float e = pick4(v, i);
+        if (look && !__builtin_isfinite(e)) {
+          const uint32_t at = row * TN + cq * 4 + i;
+          atomicOr(&map[1 + at / 32], 1u << (at & 31));
+          map[0] = 1;
+        } else {
+          store_looked_at(p, row0 + row, prob, col0 + cq * 4 + i, e, bad);
+        }
+      }
+    }
+  }
+  if (look) {
+    __syncthreads();
+    if (map[0]) {
+#pragma unroll 1
+      for (uint32_t base = 0; base < kMapWords; base += 64) {
+        // every eighth column of a row, the next one in the next row: an A
+        // row's elements and a W row's are spread over the waves alike
+        const uint32_t first = (base + lane) * 32 / TN, even = 0x01010101u << ((wave + first) & 7),
+                       odd = 0x01010101u << ((wave + first + 1) & 7);
+        const uint32_t share = TN >= 32 ? even : (even & 0xffffu) | (odd & 0xffff0000u);
+        uint32_t mine = base + lane < kMapWords ? map[1 + base + lane] & share : 0u;
+        uint64_t left;
+        while ((left = __builtin_amdgcn_ballot_w64(mine != 0)) != 0) {
+          const uint32_t l = (uint32_t)__builtin_ctzll(left);
+          const uint32_t word = (uint32_t)__builtin_amdgcn_readlane((int)mine, l);
+          const uint32_t at = (base + l) * 32 + (uint32_t)__builtin_ctz(word), row = at / TN, col = at % TN;
+          if (lane == l) mine &= mine - 1;
+          store_nonfinite(p, row0 + row, prob, col0 + col, pick4(sum4(row, col / 4), col & 3), 0, bad);
+        }
       }
     }
   }
@@ -703,9 +762,18 @@ __global__ __launch_bounds__(kThreads, 1) void tile_grid_kernel(TileParams p) {
 #pragma unroll
             for (int e = 0; e < 4; ++e) v = b == (r * NW + n) * 4 + e ? acc[n][r][e] : v;
         const uint32_t row = orow + b / (4 * NW) * 16, col = ocol + b / 4 % NW * 16 + (b & 3);
-        if (row >= p.m) continue;
-        if (__builtin_isfinite(v)) store1(p, row, prob, col, v);
-        else store_nonfinite<OP>(p, row, prob, col, v, bad);
+        const bool in = row < p.m, look = kFp8 && p.check_codes && in && !__builtin_isfinite(v);
+        if (in && !look) store_looked_at(p, row, prob, col, v, bad);
+        if constexpr (kFp8) {
+          // the wave takes its lanes' elements one after the other
+          uint64_t left = __builtin_amdgcn_ballot_w64(look);
+          while (left) {
+            const uint32_t l = (uint32_t)__builtin_ctzll(left);
+            left &= left - 1;
+            store_nonfinite(p, (uint32_t)__builtin_amdgcn_readlane((int)row, l), prob,
+                            (uint32_t)__builtin_amdgcn_readlane((int)col, l), v, l, bad);
+          }
+        }
       }
     }
   }

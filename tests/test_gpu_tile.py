@@ -209,6 +209,53 @@ def _check_grouped(out, av, w, sw, g, n):
         assert bool((err <= ref.abs() * 2.0 ** -8 + mag * k * 2.0 ** -24).all())
 
 
+# tiles of 16 x 16, 48 x 16, 80 x 64 (an odd number of row blocks, walked in
+# pairs of waves) and the walked 128 x 128
+@pytest.mark.parametrize("m,n,k", [(4, 1024, 512), (40, 1024, 2048), (301, 4096, 1024), (130, 32768, 1024)])
+def test_fp8_many_codes(eng, m, n, k):
+    """A whole A row and a whole W row of NaN codes and scattered ones: every
+    element that a wave sums again, and those beside them, are exact."""
+    import torch
+
+    a, sa, w, sw = _fp8(m, n, k, 3 * m)
+    a[m - 1], w[n // 2 + 1] = 0xFF, 0x7F
+    g = torch.Generator(device="cuda")
+    g.manual_seed(m)
+    for t, rows in ((a, m), (w, n)):
+        at = torch.randint(0, rows * k, (5,), device="cuda", generator=g)
+        t.view(-1)[at] = 0x7F
+    for out_type in (1, 2):
+        got, flag = _run_fp8(a, sa, w, sw, out_type)
+        ref = _expect(a, sa, w, sw).float()
+        assert flag == 1 and torch.equal(got, ref.bfloat16() if out_type == 1 else ref)
+
+
+@pytest.mark.parametrize("m,n,k", [(4, 1024, 4096), (64, 1024, 4096)])
+def test_fp8_code_costs_no_scan_per_element(eng, m, n, k):
+    """One NaN code in an A row makes its n sums start over: n / 16 blocks of
+    them.  Shared by the waves that is a few clean calls; a lane walking K
+    alone for each took 300 to 600 of them."""
+    import torch
+
+    a, sa, w, sw = _fp8(m, n, k, 1)
+    bad = a.clone()
+    bad[m // 2, 5] = 0xFF
+
+    def best(rows):
+        times = []
+        for _ in range(8):
+            start, stop = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            start.record()
+            _run_fp8(rows, sa, w, sw, 1)
+            stop.record()
+            stop.synchronize()
+            times.append(start.elapsed_time(stop))
+        return min(times)
+
+    best(a)
+    assert best(bad) < best(a) + 0.5
+
+
 @pytest.mark.parametrize("t", [1, 7, 65, 130])
 def test_grouped_fp8_exact(eng, t):
     """Strided problems: 4 groups of 256 x 512 over interleaved rows."""
