@@ -33,12 +33,23 @@ class engine_stream(contextlib.ContextDecorator):
     """``with engine_stream() as s``: the engine stream is torch's current
     stream inside.  The same switch as ``torch.cuda.stream(s)``; entering and
     leaving through the two calls that one ends in took 7.6 -> 1.6 us, of the
-    ~27 us of host time around a four-launch decode block."""
+    ~27 us of host time around a four-launch decode block.
+
+    A context object is entered once, as a generator's is: what to go back to
+    is kept on it, so that entered again, or by a second thread, it would
+    leave the engine stream current.  Call ``engine_stream()`` for each."""
+
+    def __init__(self) -> None:
+        self._unused = [True]
 
     def _recreate_cm(self):  # as a decorator: a context of its own per call
         return engine_stream()
 
     def __enter__(self):
+        try:
+            self._unused.pop()  # one thread gets it
+        except IndexError:
+            raise RuntimeError("pih_amd: an engine_stream() context is entered once") from None
         s = stream()
         self._other = None
         if torch._C._cuda_getDevice() != s.device_index:

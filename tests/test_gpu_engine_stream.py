@@ -35,3 +35,35 @@ def test_engine_stream_switches_and_restores():
         return depth(n - 1) if n else 0
 
     assert depth(2) == 0 and torch.cuda.current_stream() == before
+
+
+def test_engine_stream_context_is_entered_once():
+    """A second entry, from inside, afterwards or from another thread, is
+    refused and leaves every thread on the stream it had."""
+    import threading
+
+    import torch
+
+    from pih_amd.device import engine_stream, stream
+
+    before = torch.cuda.current_stream()
+    ctx, seen = engine_stream(), []
+
+    def other_thread():
+        try:
+            ctx.__enter__()
+        except RuntimeError as e:
+            seen.append((str(e), torch.cuda.current_stream() == before))
+
+    with ctx:
+        with pytest.raises(RuntimeError, match="entered once"):
+            ctx.__enter__()
+        t = threading.Thread(target=other_thread)
+        t.start()
+        t.join()
+        assert torch.cuda.current_stream() == stream()
+    assert torch.cuda.current_stream() == before and len(seen) == 1 and seen[0][1]
+    with pytest.raises(RuntimeError, match="entered once"):
+        with ctx:
+            pass
+    assert torch.cuda.current_stream() == before
