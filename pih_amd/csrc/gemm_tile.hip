@@ -201,6 +201,14 @@ struct TileShape {
   // as deep as LDS allows, at most 8 steps and 63 loads in flight
   static constexpr int kStages = std::min(std::min(kFit, 8), 63 / kLoads + 1);
   static constexpr int kParts = OP == kTileFp8 ? 2 : 4;  // waves that share an output
+  // accumulator sets a wave takes turns with, as far as registers go.  An
+  // fp32 sum of K products rounds at every MFMA, by the size it has reached:
+  // off 64 bits at K 4096 (bf16, fp32 output, normwise) 1.89e-7 with one set,
+  // 1.34e-7 with two, 1.03e-7 with four; the GEMV's 8 waves 1.37e-7, its 16
+  // waves of 2-4 rows 1.13e-7, a K split in eight 1.37e-7.  A call pays 1-2 %
+  // (4096 -> 1024 at M 8 6.0 -> 6.15 us).  (e4m3: 5.5e-5 with any number, the
+  // instruction's own rounding.)
+  static constexpr int kSets = OP == kTileFp8 ? 1 : MB == 1 && NB <= 4 ? 4 : MB * NB <= 24 ? 2 : 1;
   static constexpr uint32_t kSums = kParts * MB * NB * kSumBlock;
   static constexpr uint32_t kRing = kStages * kStage > kSums ? kStages * kStage : kSums;
 };
@@ -277,17 +285,21 @@ __global__ __launch_bounds__(kThreads, 1) void tile_gemm_kernel(TileParams p) {
     }
   }
 
-  // a wave's accumulators [W block][A block]
-  v4f acc[NW][MW];
+  // a wave's accumulators [set][W block][A block]; step j adds to set j % SETS
+  constexpr int SETS = S::kSets;
+  v4f acc[SETS][NW][MW];
 #pragma unroll
-  for (int n = 0; n < NW; ++n)
+  for (int t = 0; t < SETS; ++t)
 #pragma unroll
-    for (int r = 0; r < MW; ++r) acc[n][r] = v4f{0.f, 0.f, 0.f, 0.f};
+    for (int n = 0; n < NW; ++n)
+#pragma unroll
+      for (int r = 0; r < MW; ++r) acc[t][n][r] = v4f{0.f, 0.f, 0.f, 0.f};
   const uint32_t kh = wv & 1, half = wv >> 1;
   const uint32_t mb0 = kSplitM ? half * MW : 0, nb0 = kSplitN ? half * NW : 0;
 
-  auto compute = [&](uint32_t stage, uint32_t j, auto FF) __attribute__((always_inline)) {
+  auto compute = [&](uint32_t stage, uint32_t j, auto FF, auto SET) __attribute__((always_inline)) {
     if (kOnePair && half) return;
+    auto& sums = acc[decltype(SET)::value];
     const uint8_t* sa = smem + stage * S::kStage + (mb0 * 16 + lr) * SB;
     const uint8_t* sw = smem + stage * S::kStage + (TM + nb0 * 16 + lr) * SB;
     if constexpr (!kFp8) {
@@ -300,8 +312,8 @@ __global__ __launch_bounds__(kThreads, 1) void tile_gemm_kernel(TileParams p) {
         const v4i af = *reinterpret_cast<const v4i*>(sa + r * 4096 + at);
 #pragma unroll
         for (int n = 0; n < NW; ++n)
-          acc[n][r] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8bf, wf[n]),
-                                                              __builtin_bit_cast(v8bf, af), acc[n][r], 0, 0, 0);
+          sums[n][r] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8bf, wf[n]),
+                                                              __builtin_bit_cast(v8bf, af), sums[n][r], 0, 0, 0);
       }
     } else {
       const uint32_t at0 = ((8 * kh + lg) ^ lr) << 4, at1 = ((8 * kh + 4 + lg) ^ lr) << 4;
@@ -320,9 +332,9 @@ __global__ __launch_bounds__(kThreads, 1) void tile_gemm_kernel(TileParams p) {
         const uint32_t as = pa[(mb0 * 16 + r * 16 + lr) * KB + kb];
 #pragma unroll
         for (int n = 0; n < NW; ++n) {
-          const v4f sum = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(wf[n], af, acc[n][r], 0, 0, 0, (int)ws, 0,
+          const v4f sum = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(wf[n], af, sums[n][r], 0, 0, 0, (int)ws, 0,
                                                                            (int)as);
-          acc[n][r] = decltype(FF)::value ? without_ff_block(ws, as, acc[n][r], sum) : sum;
+          sums[n][r] = decltype(FF)::value ? without_ff_block(ws, as, sums[n][r], sum) : sum;
         }
       }
     }
@@ -372,12 +384,35 @@ __global__ __launch_bounds__(kThreads, 1) void tile_gemm_kernel(TileParams p) {
   };
   auto multiply_loop = [&](auto FF) __attribute__((always_inline)) {
     uint32_t cst = 0;
-    for (uint32_t j = 0; j < steps; ++j) {
+    auto step = [&](uint32_t j, auto SET) __attribute__((always_inline)) {
       __builtin_amdgcn_s_waitcnt(kLdsRead);
       __builtin_amdgcn_s_barrier();
-      compute(cst, j, FF);
+      compute(cst, j, FF, SET);
       cst = cst + 1 == ST ? 0 : cst + 1;
+    };
+    uint32_t j = 0;
+    for (; j + SETS <= steps; j += SETS) {
+      step(j, std::integral_constant<int, 0>{});
+      if constexpr (SETS > 1) step(j + 1, std::integral_constant<int, 1>{});
+      if constexpr (SETS > 2) {
+        step(j + 2, std::integral_constant<int, 2>{});
+        step(j + 3, std::integral_constant<int, 3>{});
+      }
     }
+    if constexpr (SETS > 1)
+      if (j < steps) step(j, std::integral_constant<int, 0>{});
+    if constexpr (SETS > 2) {
+      if (j + 1 < steps) step(j + 1, std::integral_constant<int, 1>{});
+      if (j + 2 < steps) step(j + 2, std::integral_constant<int, 2>{});
+    }
+    // the sets, pairwise
+#pragma unroll
+    for (int n = 0; n < NW; ++n)
+#pragma unroll
+      for (int r = 0; r < MW; ++r) {
+        if constexpr (SETS == 4) acc[0][n][r] = (acc[0][n][r] + acc[1][n][r]) + (acc[2][n][r] + acc[3][n][r]);
+        else if constexpr (SETS == 2) acc[0][n][r] += acc[1][n][r];
+      }
   };
   if (loader) {
     // one M tile reads each weight byte once: non-temporal, so that the A
@@ -419,7 +454,7 @@ __global__ __launch_bounds__(kThreads, 1) void tile_gemm_kernel(TileParams p) {
 #pragma unroll
     for (int r = 0; r < MW; ++r)
       *reinterpret_cast<v4f*>(smem + (part * MB * NB + (mb0 + r) * NB + nb0 + n) * kSumBlock + lg * kSumGroup + lr * 16) =
-          acc[n][r];
+          acc[0][n][r];
   __syncthreads();
   constexpr uint32_t QR = TN / 4;  // 4-column groups per row
   // columns 4 cq .. + 3 of a row, summed over the waves
@@ -499,6 +534,11 @@ struct GridShape {
   // three of them ahead spilled (128 x 128 tiles: 23.3 -> 25.5 us at M 2048,
   // 4096 -> 2048; bf16 256 x 128: 60.6 -> 57.2 us at 4096 -> 4096 with three)
   static constexpr int kAhead = OP == kTileBf16 ? 3 : 1;
+  // accumulator sets (see TileShape): the two 32-k slices of a bf16 step each
+  // have one where registers hold them; 12 and 16 row blocks (96 and 128
+  // accumulator registers a set) have one chain, the rounding of an unsplit
+  // sum on the 128 x 256 tiles
+  static constexpr int kSets = OP == kTileBf16 && MB == 8 ? 2 : 1;
 };
 
 template <int OP, int MB, int NB, int SBW>
@@ -644,11 +684,14 @@ __global__ __launch_bounds__(kThreads, 1) void tile_grid_kernel(TileParams p) {
   for (uint32_t i = 0; i < tiles; ++i) {
     uint32_t row0, col0, prob;
     tile_at(i, row0, col0, prob);
-    v4f acc[NW][MW];
+    v4f sums[S::kSets][NW][MW];
 #pragma unroll
-    for (int n = 0; n < NW; ++n)
+    for (int t = 0; t < S::kSets; ++t)
 #pragma unroll
-      for (int r = 0; r < MW; ++r) acc[n][r] = v4f{0.f, 0.f, 0.f, 0.f};
+      for (int n = 0; n < NW; ++n)
+#pragma unroll
+        for (int r = 0; r < MW; ++r) sums[t][n][r] = v4f{0.f, 0.f, 0.f, 0.f};
+    auto& acc = sums[0];
     const uint8_t* const pan = panels + (i & 1) * S::kPanelOne;
     // step j, whose first slice's W fragments are in wf[P]
     auto step = [&](uint32_t j, auto PAR, auto FF) __attribute__((always_inline)) {
@@ -674,8 +717,8 @@ __global__ __launch_bounds__(kThreads, 1) void tile_grid_kernel(TileParams p) {
                                                                              0, (int)sa);
             acc[n][r] = decltype(FF)::value ? without_ff_block(sw, sa, acc[n][r], sum) : sum;
           } else {
-            acc[n][r] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8bf, wf[wb][n]),
-                                                                __builtin_bit_cast(v8bf, a), acc[n][r], 0, 0, 0);
+            sums[q % S::kSets][n][r] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                __builtin_bit_cast(v8bf, wf[wb][n]), __builtin_bit_cast(v8bf, a), sums[q % S::kSets][n][r], 0, 0, 0);
           }
         }
         __builtin_amdgcn_sched_barrier(0);
@@ -709,6 +752,12 @@ __global__ __launch_bounds__(kThreads, 1) void tile_grid_kernel(TileParams p) {
     };
     if (kFp8 && ff) run(std::true_type{});
     else run(std::false_type{});
+    if constexpr (S::kSets == 2) {
+#pragma unroll
+      for (int n = 0; n < NW; ++n)
+#pragma unroll
+        for (int r = 0; r < MW; ++r) acc[n][r] += sums[1][n][r];
+    }
     const uint32_t orow = row0 + wm * MW * 16 + lr, ocol = col0 + wn * NW * 16 + 4 * lg;
     bool nonfin = false;
 #pragma unroll

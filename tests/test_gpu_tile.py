@@ -57,6 +57,31 @@ def test_bf16_exact(eng, m, n, k):
     assert torch.equal(b16, ref.float().bfloat16())
 
 
+# 16 x 16 (four accumulator sets in each of four waves), 48 x 64 and 80 x 64
+# (two in each) and the walked 128 x 128 (two)
+@pytest.mark.parametrize("m,n,k,chains,limit", [(3, 1024, 4096, 16, 1.2e-7), (130, 4096, 4096, 8, 1.6e-7),
+                                                (300, 4096, 4096, 8, 1.6e-7), (1024, 4096, 4096, 2, 3.3e-7)])
+def test_bf16_rounding_of_the_sums(eng, m, n, k, chains, limit):
+    """Normwise error of fp32 outputs against 64 bits.  A chain of c MFMAs
+    rounds each time by up to 2^-24 of what it has reached, in sum about
+    2^-24 sqrt(c / 6) of its result (c = k / 32 / chains); measured 1.03e-7,
+    1.34e-7 and 2.7e-7, and sqrt(2) times that with half the chains, which the
+    limits leave out."""
+    import torch
+
+    from pih_amd.linear import bf16_gemm
+
+    g = torch.Generator(device="cuda")
+    g.manual_seed(m)
+    a = torch.randn(m, k, device="cuda", generator=g).bfloat16()
+    w = (torch.randn(n, k, device="cuda", generator=g) * 0.02).bfloat16()
+    got = bf16_gemm(a, w, abi.OUTPUT_F32)
+    torch.cuda.synchronize()
+    ref = a.double() @ w.double().T
+    err = ((got.double() - ref).norm() / ref.norm()).item()
+    assert 2.0 ** -24 * (k / 32 / chains / 6) ** 0.5 * 0.5 < err < limit
+
+
 @pytest.mark.parametrize("m,n,k", [(5, 64, 256), (40, 128, 384)])
 def test_bf16_unaligned_operand(eng, m, n, k):
     """W 8 bytes off a 16-byte boundary: the GEMV the call took before."""
