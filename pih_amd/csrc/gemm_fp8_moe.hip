@@ -1773,14 +1773,7 @@ St LaunchBigTileGemm(const BigTileArgs& a, bool* codes_in_tiles) {
   mp.experts = splits > 1 ? splits : a.problems;
   mp.k_splits = splits;
   mp.a_rows_total = (uint32_t)a_rows;
-  // fewer 128-row tiles than about a round on the CUs (and no K split):
-  // 64- or 32-row M tiles, up to four times the tiles at the same K depth
-  // (same arithmetic per element; the tiles stream their W tile from L2)
-  uint32_t tile_rows = BM;
-  if (splits == 1) {
-    const uint64_t nt = (a.n + BN - 1) / BN;
-    while (tile_rows > 32 && (uint64_t)((a.m + tile_rows - 1) / tile_rows) * nt * a.problems < 192) tile_rows /= 2;
-  }
+  const uint32_t tile_rows = DenseTileRows(a.m, a.n, a.problems, splits);
   mp.dense_tile_rows = tile_rows;
   mp.dense_m_tiles = (a.m + tile_rows - 1) / tile_rows;
   mp.a_row_stride = a.a_row_stride;
@@ -1872,22 +1865,6 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float* __restr
 }
 
 }  // namespace
-
-uint32_t DenseKSplits(uint32_t m, uint32_t n, uint32_t k_steps) {
-  // a split is worth it below one 128 x 256 tile per CU (256 CUs); the
-  // smallest split count that reaches a full round, with at least 8 K steps
-  // per split, else the largest such count (a GEMM of few tiles: M 128,
-  // 12288 -> 4096 has 16)
-  const uint64_t tiles = (uint64_t)((m + BM - 1) / BM) * ((n + BN - 1) / BN);
-  if (tiles == 0 || tiles >= 192) return 1;
-  uint32_t best = 1;
-  for (uint32_t s = 2; s <= 8; ++s) {
-    if (k_steps % s || k_steps / s < 8) continue;
-    if (tiles * s >= 192) return s;
-    best = s;
-  }
-  return best;
-}
 
 St LaunchSplitKReduce(const float* ws, uint32_t splits, uint32_t m, uint32_t n, void* out, OutKind out_kind,
                       uint32_t* err, uint32_t bit, hipStream_t stream) {

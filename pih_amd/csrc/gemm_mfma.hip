@@ -760,15 +760,16 @@ St LaunchFp8BlockGemm(const BlockGemmArgs& a) {
   const bool dense_ok = !a.moe && !a.a_gather && (a.out_kind == kOutBf16 || a.out_kind == kOutF32) &&
                         (contiguous1 || !a.check_codes) && (uint64_t)a.a_rows_total * a.k <= 0xffffffffull &&
                         (uint64_t)a.n * a.k <= 0xffffffffull;
-  // UE8M0 scales: tiles chosen per shape from one row up (gemm_tile.hip), in
-  // place of the small-M kernel and of the 128 x 256 tiles.  DeepSeek
-  // launch_fp8_gemm, K -> N, us before -> after (one MI355X, weights rotated
-  // past the caches), M 4 / 64 / 301 / 2048:
-  //   4096 -> 1024   5.8 -> 4.2    15.4 -> 4.8    28.6 -> 6.8    31 -> 15.4
-  //   1024 -> 32768  9.8 -> 7.4    15.0 -> 9.5    32.6 -> 24.1   134 -> 114
-  //   8192 -> 4096   10.9 -> 7.7   29.5 -> 12.4   50.2 -> 22.5   78 -> 80
-  //   4096 -> 2048   6.0 -> 4.8    15.5 -> 5.9    29.0 -> 9.2    34 -> 23.3
-  //   2048 -> 4096   5.0 -> 4.3    8.9 -> 5.6     18.4 -> 8.2    29.5 -> 27.3
+  const bool big = Fp8BigTiles(a.m, a.n, a.k, a.problems);
+  // UE8M0 scales: tiles chosen per shape from one row up (gemm_tile.hip), with
+  // the exceptions of Fp8OnTiles.  DeepSeek launch_fp8_gemm, K -> N, us without
+  // -> with them (one MI355X, weights rotated past the caches), M 4 / 64 / 301
+  // / 2048:
+  //   4096 -> 1024   5.8 -> 4.3    15.3 -> 4.9    26.1 -> 7.1    27.2 -> 15.5
+  //   1024 -> 32768  10.0 -> 8.2   15.3 -> 9.8    33.1 -> 22.2   127 -> 101
+  //   8192 -> 4096   11.2 -> 8.0   30.4 -> 13.2   51.5 -> 23.1   77 (128 x 256)
+  //   4096 -> 2048   5.9 -> 4.6    15.6 -> 6.4    28.8 -> 9.8    33.1 -> 23.2
+  //   2048 -> 4096   4.5 -> 4.1    8.9 -> 5.5     18.8 -> 8.9    27.9 -> 25.5
   if (dense_ok && a.scale_fmt == kScaleUe8m0) {
     TileGemmArgs t;
     t.a = a.a;
@@ -793,29 +794,11 @@ St LaunchFp8BlockGemm(const BlockGemmArgs& a) {
     t.err_scale_bit = a.err_scale_bit;
     t.err_nonfinite_bit = a.err_nonfinite_bit;
     t.write_nonfinite = a.write_nonfinite;
-    if (TileGemmTakes(t)) return LaunchTileGemm(t);
-  }
-  // Above 64 rows the big tiles also take what the 128 x 128 kernel took
-  // before (more than 256 rows, or too many 128 x 128 tiles for the small-M
-  // kernel) and the small-M kernel's 64-row chunks once together they would
-  // stream more than 20 MB of weights (each chunk streams all of W).
-  // DeepSeek launch_fp8_gemm, K -> N at M rows, us before -> after:
-  // 4096 -> 1024 M 384 63 -> 26; 8192 -> 4096 M 128 56 -> 50, M 256 111 ->
-  // 50, M 384 122 -> 51; 4096 -> 2048 M 192 30 -> 27, M 512 63 -> 28;
-  // 2048 -> 4096 M 256 26 -> 18; 1024 -> 32768 M 100 22 -> 17.  Below
-  // those sizes the small-M kernel stays faster (4096 -> 1024 at M 256: 16
-  // against 26 us: a big tile's 32 K steps take ~0.8 us each).
-  // At 33..64 rows the big tiles also win where the small-M kernel's one
-  // pass over W (~1.15 TB/s at 64 rows) takes longer than a round of big
-  // tiles (~0.8 us per 128-deep K step + ~5 us): 1024 -> 32768 at M 64,
-  // 25 -> 16 us.
-  bool big = BigTileWorthIt(a.m, a.n * a.problems);
-  const uint64_t w_bytes = (uint64_t)a.n * a.k * a.problems;
-  if (a.m > kSmallMChunkRows) {
-    const uint64_t chunks = (a.m + kSmallMChunkRows - 1) / kSmallMChunkRows;
-    big = big || a.m > kSmallMRows || !SmallMTakes(a.m, a.n, a.problems) || chunks * w_bytes > (20ull << 20);
-  } else if (a.m > 32) {
-    big = big || w_bytes / 1150 > (uint64_t)(a.k / 128) * 800 + 5000;  // ns
+    if (TileGemmTakes(t)) {
+      const TilePick tile = PickTile(false, a.m, a.n, a.k, a.problems);
+      if (Fp8OnTiles(a.m, a.n, a.k, a.problems, a.out_kind == kOutF32, a.check_codes, big, tile))
+        return LaunchTileGemm(t, tile);
+    }
   }
   const bool dense1 = dense_ok && big;
   if (dense1) {
@@ -991,25 +974,25 @@ St LaunchBf16Gemm(const Bf16GemmArgs& a) {
   if (!a.a || !a.w || !a.out || !a.stream) return Invalid("bf16_gemm_null_argument");
   if (a.m == 0 || a.n == 0 || a.k == 0) return Invalid("bf16_gemm_shape_invalid");
   if (a.out_kind != kOutBf16 && a.out_kind != kOutF32) return Invalid("bf16_gemm_output_type_invalid");
-  // Batches of 2..255 rows against very wide weights (the LM heads: a round
-  // of 256-column tiles without a K split) take the big tiles, which stream
-  // the weights once (twice through L2 above 128 rows) with the batch in one
-  // M tile, where the GEMV re-reads the batch's rows from L2 for every 16
-  // weight rows and the 128 x 128 kernel is MFMA-bound on its small tiles
-  // (DeepSeek LM head, 4096 -> 129280: m = 2 186 -> 165 us, m = 16 194 ->
-  // 170 us, m = 64 177 us, m = 128 233 -> 186 us, m = 200 364 -> 285 us;
-  // m = 1 stays on the GEMV, 159 us).
-  const bool wide = a.m >= 2 && a.m < 256 && a.n % 128 == 0 && a.k % 64 == 0 && a.n / 256 >= 192;
-  // Tiles chosen per shape (gemm_tile.hip) from two rows up; one row, and
-  // very wide weights up to 128 rows (HBM-bound on the big tiles: 6.1 TB/s),
-  // stay where they are.  Qwen3-8B projections, K -> N, us before -> after at
-  // M 2 / 17 / 57 / 200 / 2048 (one MI355X, weights rotated past the caches):
-  //   4096 -> 4096   8.5 -> 7.8    10.9 -> 8.3   14.3 -> 11.3   25 -> 16   63 -> 57
-  //   4096 -> 1024   6.2 -> 6.1    9.1 -> 6.0    12.8 -> 6.1    21 -> 8.1  33 -> 28
-  //   4096 -> 12288  20.4 -> 16.5  21.9 -> 18.7  30.5 -> 21.3   47 -> 38   182 -> 165
-  //   12288 -> 4096  17.3 -> 17.7  23.5 -> 20.4  37 -> 29       48 -> 43   182 -> 160
-  // (above 64 rows only what was taken there: whole 128-column groups)
-  if (a.m >= 2 && (a.m <= 64 || a.n % 128 == 0) && (!wide || a.m > 128)) {
+  const bool wide = Bf16Wide(a.m, a.n, a.k);
+  const bool big = (Bf16BigTiles(a.m, a.n, a.k) || wide) && (uint64_t)a.m * a.k * 2 <= 0xffffffffull &&
+                   (uint64_t)a.n * a.k * 2 <= 0xffffffffull;
+  // fewer big tiles than CUs: K split into fp32 partial sums in the caller's
+  // workspace (sized by Bf16GemmWorkspaceBytes), then summed in split order;
+  // the reduce stores 8 or 16 bytes per lane, so the workspace and the output
+  // must start on 16-byte boundaries (torch allocations do)
+  uint32_t splits = a.k % 64 ? 1 : DenseKSplits(a.m, a.n, a.k / 64);
+  if (!a.workspace || a.workspace_bytes < (uint64_t)splits * a.m * a.n * 4 ||
+      (reinterpret_cast<uintptr_t>(a.workspace) | reinterpret_cast<uintptr_t>(a.out)) % 16)
+    splits = 1;
+  // Tiles chosen per shape (gemm_tile.hip), with the exceptions of Bf16OnTiles.
+  // Qwen3-8B projections, K -> N, us without -> with them at M 2 / 17 / 57 / 200
+  // / 2048 (one MI355X, weights rotated past the caches):
+  //   4096 -> 4096   8.7 -> 7.8    10.3 -> 8.8   13.0 -> 12.0   25.0 -> 17.3   63 -> 57
+  //   4096 -> 1024   5.9 -> 5.7    8.0 -> 5.9    11.0 -> 6.4    21.3 -> 9.3    31 -> 29
+  //   4096 -> 12288  20.3 -> 17.7  22.6 -> 19.8  31.0 -> 22.8   45.7 -> 39.0   183 -> 163
+  //   12288 -> 4096  18.7 -> 18.7  24.8 -> 21.6  34.0 -> 31.8   46 (K split)   175 -> 160
+  if (a.m >= 2) {
     TileGemmArgs t;
     t.a = a.a;
     t.w = a.w;
@@ -1027,12 +1010,14 @@ St LaunchBf16Gemm(const Bf16GemmArgs& a) {
       t.err_nonfinite_bit = a.nonfinite_bit;
     }
     t.write_nonfinite = true;
-    if (TileGemmTakes(t)) return LaunchTileGemm(t);
+    if (TileGemmTakes(t)) {
+      const TilePick tile = PickTile(true, a.m, a.n, 2 * a.k, 1);
+      if (Bf16OnTiles(a.m, a.n, a.k, a.out_kind == kOutF32, big, splits, tile)) return LaunchTileGemm(t, tile);
+    }
   }
   if (a.m <= 64 && !wide) return LaunchBf16Gemv(a);
   if (a.n % 128 || a.k % 64) return Invalid("bf16_gemm_shape_invalid");
-  if ((Bf16BigTiles(a.m, a.n, a.k) || wide) && (uint64_t)a.m * a.k * 2 <= 0xffffffffull &&
-      (uint64_t)a.n * a.k * 2 <= 0xffffffffull) {
+  if (big) {
     BigTileArgs b;
     b.a = a.a;
     b.w = a.w;
@@ -1051,15 +1036,7 @@ St LaunchBf16Gemm(const Bf16GemmArgs& a) {
       b.err_nonfinite_bit = a.nonfinite_bit;
     }
     b.write_nonfinite = true;
-    // fewer tiles than CUs: K split into fp32 partial sums in the caller's
-    // workspace (sized by Bf16GemmWorkspaceBytes), then summed in split
-    // order; the reduce stores 8 or 16 bytes per lane, so the workspace and
-    // the output must start on 16-byte boundaries (torch allocations do)
-    const uint32_t splits = DenseKSplits(a.m, a.n, a.k / 64);
-    const uint64_t ws_bytes = (uint64_t)splits * a.m * a.n * 4;
-    const bool aligned =
-        reinterpret_cast<uintptr_t>(a.workspace) % 16 == 0 && reinterpret_cast<uintptr_t>(a.out) % 16 == 0;
-    if (splits > 1 && a.workspace && a.workspace_bytes >= ws_bytes && aligned) {
+    if (splits > 1) {
       BigTileArgs p = b;
       p.out = a.workspace;
       p.out_kind = kOutF32;

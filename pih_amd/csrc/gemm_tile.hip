@@ -46,8 +46,7 @@ namespace {
 
 enum : int { kTileBf16 = 0, kTileFp8 = 1 };
 constexpr uint32_t SB = 256;  // bytes of a row per K step
-constexpr uint32_t kGridStep = 128;  // ... in the kernel that walks tiles
-constexpr uint32_t kCus = 256;
+constexpr uint32_t kGridStep = kWalkStep;  // ... in the kernel that walks tiles
 constexpr uint32_t kThreads = 512;  // waves 0-3 multiply, waves 4-7 load
 constexpr uint32_t kMaxKb = 64;  // e4m3: K / 128 the scale panels hold
 constexpr uint32_t kOutPitch = 144;  // staged output rows: 128 bytes + 16
@@ -881,51 +880,6 @@ void launch_pick(const TilePick& t, const TileParams& p, hipStream_t s) {
 
 }  // namespace
 
-// The tile for a shape, by an estimate of its time: the rounds of tiles on the
-// CUs times what a CU loads for one (at the ~64 GB/s it takes in while part of
-// its lines come from HBM), no less than the weights at the 6.2 TB/s they
-// stream at, and 1.5 us for each round after the first (the start-up that the
-// tile-walking kernel hides).  16 x 16 tiles share a CU two at a time: their
-// weights were measured to stream at 7 TB/s (12288 x 4096 bf16 at m 8: 16.5
-// us, 18.4 with 16 x 48 tiles) and a round is 512 of them, 1.1 us apart.
-// Over 100 shapes (m 1-2048; Qwen3-8B, Qwen3 MLP and DeepSeek projections) the
-// choice was the fastest measured tile or within 13 % of it, 1 % on average.
-TilePick PickTile(bool bf16, uint32_t m, uint32_t n, uint32_t row_bytes, uint32_t problems) {
-  TilePick best;
-  double best_ns = 0.0;
-  const double w_bytes = (double)n * problems * row_bytes;
-  auto consider = [&](uint32_t mb, uint32_t nb, bool grid) {
-    if (n % (16 * nb) || (mb > 1 && 16 * (mb - 1) >= m && mb < 8)) return;
-    const uint64_t tiles = (uint64_t)((m + 16 * mb - 1) / (16 * mb)) * (n / (16 * nb)) * problems;
-    const bool paired = mb == 1 && nb == 1;
-    const double rounds = (double)((tiles + kCus - 1) / kCus);
-    const double load = rounds * 16.0 * (mb + nb) * row_bytes / 64.0;
-    const double hbm = w_bytes / (paired ? 7000.0 : 6200.0);
-    const double start = grid     ? 0.0
-                         : paired ? (double)((tiles + 2 * kCus - 1) / (2 * kCus) - 1) * 1100.0
-                                  : (rounds - 1.0) * 1500.0;
-    const double ns = std::max(load, hbm) + start + 0.02 * load;
-    // as good: the more nearly square tile, then the taller one
-    const bool tie = ns < best_ns + 1e-6 && (std::min(mb, nb) > std::min(best.mb, best.nb) ||
-                                             (std::min(mb, nb) == std::min(best.mb, best.nb) && mb > best.mb));
-    if (!best.mb || ns < best_ns - 1e-6 || tie) {
-      best = TilePick{mb, nb, grid};
-      best_ns = ns;
-    }
-  };
-  for (uint32_t mb : {1u, 2u, 3u, 4u, 5u, 6u, 8u})
-    for (uint32_t nb : {1u, 2u, 3u, 4u, 8u})
-      if ((bf16 || nb != 3) && (nb != 8 || mb <= 4)) consider(mb, nb, false);
-  // (a tile's scale panel is reused two tiles later: the ring must not run
-  // further ahead than one tile)
-  if (row_bytes / kGridStep >= 8) {
-    consider(8, 8, true);
-    consider(12, 8, true);
-    if (bf16) consider(16, 8, true);
-  }
-  return best;
-}
-
 bool TileGemmTakes(const TileGemmArgs& a) {
   const uint64_t rb = a.bf16 ? 2ull * a.k : a.k, osz = a.out_kind == kOutF32 ? 4 : 2;
   if (a.m == 0 || a.n == 0 || a.k == 0 || a.problems == 0 || rb % SB || a.n % (a.bf16 ? 16 : 128)) return false;
@@ -943,7 +897,7 @@ bool TileGemmTakes(const TileGemmArgs& a) {
          (reinterpret_cast<uintptr_t>(a.a_scale) | reinterpret_cast<uintptr_t>(a.w_scale)) % 4 == 0;
 }
 
-St LaunchTileGemm(const TileGemmArgs& a) {
+St LaunchTileGemm(const TileGemmArgs& a, const TilePick& t) {
   if (!a.a || !a.w || !a.out || !a.stream || (!a.bf16 && (!a.a_scale || !a.w_scale || !a.error_flag)))
     return Invalid("tile_gemm_null_argument");
   if (!TileGemmTakes(a)) return Invalid("tile_gemm_shape_invalid");
@@ -970,7 +924,6 @@ St LaunchTileGemm(const TileGemmArgs& a) {
     p.err_scale = a.err_scale_bit;
     p.err_nonfinite = a.err_nonfinite_bit;
   }
-  const TilePick t = PickTile(a.bf16, a.m, a.n, p.row_bytes, a.problems);
   St s = RequireCleanLastError();
   if (!s.ok()) return s;
   if (a.bf16) launch_pick<kTileBf16>(t, p, a.stream);

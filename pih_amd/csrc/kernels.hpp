@@ -8,6 +8,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "dense_route.hpp"
 #include "host_common.hpp"
 
 namespace pih_amd {
@@ -115,11 +116,6 @@ St LaunchFp4Gemm(const Fp4GemmArgs& a);
 // tiles (too few blocks to stream the weights).  `taken` is false when it
 // does not take the shape (the caller then uses the tiled kernel); the
 // callers' checks come first.
-constexpr uint32_t kSmallMChunkRows = 64, kSmallMRows = 256;
-inline bool SmallMTakes(uint32_t m, uint32_t n, uint32_t problems) {
-  if (m <= kSmallMChunkRows) return m > 0;
-  return m <= kSmallMRows && (uint64_t)((m + 127) / 128) * ((n + 127) / 128) * problems < 128;
-}
 St LaunchFp8SmallM(const BlockGemmArgs& a, bool& taken);
 St LaunchFp4SmallM(const Fp4GemmArgs& a, bool& taken);
 // MoE problems: experts with at most Fp4MoeLightRows(a) rows (64; 0 when
@@ -221,17 +217,7 @@ struct TileGemmArgs {
   bool write_nonfinite = false;
 };
 bool TileGemmTakes(const TileGemmArgs& a);
-St LaunchTileGemm(const TileGemmArgs& a);
-// The tile it runs: 16 mb x 16 nb output elements, one per block or (grid)
-// one block per CU walking them
-struct TilePick {
-  uint32_t mb = 0, nb = 0;
-  bool grid = false;
-};
-TilePick PickTile(bool bf16, uint32_t m, uint32_t n, uint32_t row_bytes, uint32_t problems);
-// K splits for a dense big-tile GEMM of k_steps 128-byte K steps (1: none):
-// below a round of tiles on the 256 CUs
-uint32_t DenseKSplits(uint32_t m, uint32_t n, uint32_t k_steps);
+St LaunchTileGemm(const TileGemmArgs& a, const TilePick& tile);
 // out[m, n] = sum over the splits in order of ws[q][m][n] (bf16 or fp32)
 St LaunchSplitKReduce(const float* ws, uint32_t splits, uint32_t m, uint32_t n, void* out, OutKind out_kind,
                       uint32_t* err, uint32_t bit, hipStream_t stream);
@@ -249,20 +235,6 @@ struct NanCodeScanArgs {
   hipStream_t stream = nullptr;
 };
 St LaunchNanCodeScan(const NanCodeScanArgs& a);
-// the big-tile path pays from 64 tiles on (measured at M = 2048: N = 1024,
-// 64 tiles on 64 CUs, 40.7 us against 64 us for the 128 x 128 kernel's 128
-// tiles)
-inline bool BigTileWorthIt(uint32_t m, uint32_t n) {
-  return m >= 256 && (uint64_t)((m + 127) / 128) * ((n + 255) / 256) >= 64;
-}
-// BF16 GEMMs above 64 rows take the big tiles (K split into the queried
-// workspace when their tiles are few) from 512-deep K and 256 columns on:
-// against the 128 x 128 kernel, Qwen3-8B projections at M 65-384 ran
-// 1.3-3.8x faster (4096 -> 4096 M 192 64 -> 25 us, 12288 -> 4096 M 192
-// 181 -> 47 us, 4096 -> 1024 M 1024 58 -> 28 us) and nowhere slower.
-inline bool Bf16BigTiles(uint32_t m, uint32_t n, uint32_t k) {
-  return BigTileWorthIt(m, n) || (m > 64 && k >= 512 && n >= 256);
-}
 uint64_t Bf16GemmWorkspaceBytes(uint32_t m, uint32_t n, uint32_t k);
 // decode shapes (m <= 64): the weight-streaming GEMV with split-K
 St LaunchBf16Gemv(const Bf16GemmArgs& a);

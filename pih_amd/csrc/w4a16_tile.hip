@@ -30,7 +30,7 @@
 namespace pih_amd {
 namespace {
 
-constexpr uint32_t kThreads = 512, kCus = 256, kMaxGroup = 8;
+constexpr uint32_t kThreads = 512, kMaxGroup = 8;
 constexpr uint32_t kMaxGroups = 96;  // K / 128 the panels hold
 constexpr uint32_t kReservedNibble = 12, kBadScale = 13, kNonFinite = 14;
 

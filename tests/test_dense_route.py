@@ -1,0 +1,93 @@
+"""The rules of dense_route.hpp, compiled for the CPU: which kernel a dense
+GEMM runs on and its tile.
+
+* every tile that the rules choose over the shapes of the models here and over
+  generic ones is one the kernels are built for;
+* calls measured on both kernels (one MI355X, us) go to the faster one,
+  wherever the two are 5 % apart or more."""
+import ctypes
+import os
+import shutil
+import subprocess
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+CSRC = os.path.join(os.path.dirname(HERE), "pih_amd", "csrc")
+
+# (N, K): Qwen3-8B, the Qwen3 MLP blocks and the LM heads; DeepSeek FP8
+QWEN = [(4096, 4096), (1024, 4096), (12288, 4096), (4096, 12288)]
+MLP = [(3 * h, h) for h in (1024, 2048, 2560)] + [(h, 3 * h) for h in (1024, 2048, 2560)]
+HEADS = [(129280, 4096), (151936, 1024), (151936, 2560), (151936, 4096)]
+DEEPSEEK = [(1024, 4096), (32768, 1024), (4096, 8192), (2048, 4096), (4096, 2048)]
+ROWS = sorted(set(range(1, 129)) | set(range(129, 2049, 7)) | {256, 512, 1024, 1500, 2047, 2048, 4096})
+
+
+@pytest.fixture(scope="module")
+def route(tmp_path_factory):
+    if shutil.which("g++") is None:
+        pytest.skip("needs g++")
+    lib = str(tmp_path_factory.mktemp("route") / "route.so")
+    subprocess.run(["g++", "-O2", "-std=c++17", "-shared", "-fPIC", "-Wall", "-Werror", "-I", CSRC,
+                    os.path.join(HERE, "dense_route_check.cpp"), "-o", lib], check=True)
+    return ctypes.CDLL(lib)
+
+
+def _tile(route, bf16, m, n, k, problems=1):
+    v = route.pick_tile(int(bf16), m, n, k, problems)
+    return v & 0xFF, v >> 8 & 0xFF, v >> 16
+
+
+def _built(bf16):
+    one = {(mb, nb, 0) for mb in (1, 2, 3, 4, 5, 6, 8) for nb in (1, 2, 3, 4, 8)
+           if (bf16 or nb != 3) and (nb != 8 or mb <= 4)}
+    return one | {(8, 8, 1), (12, 8, 1)} | ({(16, 8, 1)} if bf16 else set())
+
+
+@pytest.mark.parametrize("bf16", [True, False])
+def test_only_built_tiles_are_chosen(route, bf16):
+    step = 16 if bf16 else 128
+    generic = [(n, k) for n in (step, 3 * step, 128, 384, 640, 1280, 5120, 28672)
+               for k in ((128, 256, 384, 640, 5120, 17408) if bf16 else (512, 1024, 1536, 7168, 8192))]
+    for n, k in generic + (QWEN + MLP + HEADS if bf16 else DEEPSEEK):
+        for m in ROWS:
+            for problems in (1,) if bf16 else (1, 4, 8):
+                tile = _tile(route, bf16, m, n, k, problems)
+                assert tile in _built(bf16), (m, n, k, problems, tile)
+                # a walked tile has at least 8 K steps; a tile's columns divide n
+                assert n % (16 * tile[1]) == 0 and (not tile[2] or (2 * k if bf16 else k) >= 1024)
+
+
+# (m, n, k, us on the other kernel, us on the tiles)
+FP8_MEASURED = [
+    (1, 128, 512, 2.67, 2.98), (2, 256, 512, 2.75, 3.15), (8, 2048, 512, 3.07, 3.31), (1, 4096, 1024, 3.45, 3.72),
+    (1, 129280, 1024, 27.2, 33.8), (8, 7168, 512, 3.9, 3.5), (4, 1024, 4096, 5.77, 4.27), (4, 32768, 1024, 10.0, 8.1),
+    (64, 4096, 8192, 30.4, 13.2), (301, 32768, 1024, 33.1, 22.2), (2048, 1024, 4096, 27.2, 15.5),
+    (4096, 32768, 512, 169.6, 313.0), (2048, 16384, 512, 46.6, 78.8), (4096, 7168, 512, 46.1, 66.9),
+    (4096, 2048, 7168, 66.7, 80.8), (4096, 2048, 4096, 44.3, 50.7), (2048, 4096, 8192, 76.1, 80.2),
+    (2048, 4096, 6144, 60.1, 64.9), (4096, 8192, 8192, 284.6, 309.6), (2048, 12288, 4096, 121.6, 128.5),
+    (512, 4096, 8192, 50.5, 29.3), (1024, 2048, 7168, 47.5, 26.0), (2048, 32768, 1024, 127.0, 101.0)]
+BF16_MEASURED = [
+    (8, 1024, 128, 2.08, 2.77), (8, 1024, 1024, 3.35, 3.55), (16, 3072, 1024, 3.85, 4.05), (8, 256, 512, 2.5, 3.0),
+    (8, 1024, 768, 3.7, 3.1), (2, 12288, 4096, 20.3, 17.7),
+    (17, 12288, 4096, 21.6, 18.7), (57, 1024, 4096, 11.0, 6.4), (200, 4096, 4096, 25.0, 17.3),
+    (200, 28672, 4096, 87.0, 78.0), (2048, 12288, 4096, 183.0, 163.0), (2048, 4096, 12288, 175.0, 160.0),
+    (4096, 1024, 16384, 119.4, 257.1), (2048, 1024, 16384, 68.9, 121.5), (2048, 256, 16384, 42.5, 77.0),
+    (4096, 512, 7168, 41.2, 66.7), (1024, 2560, 7680, 52.4, 72.0), (256, 4096, 12288, 49.9, 59.4),
+    (1024, 4096, 12288, 103.0, 118.3), (200, 8192, 28672, 130.5, 189.7), (128, 5120, 17408, 52.0, 69.2),
+    (4096, 4096, 256, 22.3, 36.4), (1000, 5120, 5120, 90.7, 52.4), (2048, 2560, 7680, 125.3, 82.7)]
+
+
+def test_measured_calls_go_to_the_faster_kernel(route):
+    for m, n, k, other, tiles in FP8_MEASURED:
+        assert bool(route.fp8_on_tiles(m, n, k, 1, 0, 1)) == (tiles < other), ("fp8", m, n, k)
+    for m, n, k, other, tiles in BF16_MEASURED:
+        assert bool(route.bf16_on_tiles(m, n, k, 0, 1)) == (tiles < other), ("bf16", m, n, k)
+
+
+def test_grouped_calls_stay_off_the_128_x_256_tiles(route):
+    """Without a code check those read blocks under a 0xFF weight scale."""
+    for m in (64, 257, 700, 2048, 4096):
+        for n, k in ((1024, 4096), (128, 512), (4096, 8192)):
+            for problems in (1, 4, 8, 16):
+                assert route.fp8_on_tiles(m, n, k, problems, 0, 0)
