@@ -213,4 +213,52 @@ inline bool Bf16OnTiles(uint32_t m, uint32_t n, uint32_t k, bool f32_out, bool b
   return m <= 64 || !big || !BigTilesFaster(true, m, n, k, 1, f32_out, t, k_splits);
 }
 
+// W4A16 (w4a16_tile.hip), count problems of n[i] rows, shapes that it runs (k %
+// 512 == 0): the 16-row weight blocks of a tile, or 0 for the GEMV kernels.  By
+// measurement (one MI355X, asymmetric, us GEMV -> here; blocks: 16-row weight
+// blocks of the launch):
+//   K 4096, 384 blocks      m 2   6.1 -> 7.5    m 8   9.2 -> 7.2    m 16  10.1 -> 7.3   m 32  17.2 -> 9.3
+//   K 4096, 256 blocks      m 2   4.8 -> 5.9    m 9   5.30 -> 5.55  m 16  5.9 -> 5.6    m 32  9.5 -> 8.0
+//   K 4096, 1536 blocks     m 2   15.5 -> 13.1  m 8   16.9 -> 13.7  m 16  18.0 -> 13.8  m 32  49 -> 17.7
+//   K 12288, 256 blocks     m 2   8.8 -> 11.9   m 9   11.0 -> 10.5  m 16  12.9 -> 10.9  m 32  21.8 -> 17.0
+//   K 2048, 768 blocks      m 2   5.54 -> 6.10  m 4   6.3 -> 6.1    m 16  7.3 -> 6.4    m 32  16.2 -> 8.0
+//   K 4096, 16 blocks       m 9   4.96 -> 5.10  m 12  5.08 -> 5.15  m 16  5.32 -> 5.20  m 32  8.7 -> 7.4
+//   K 2048, 128 blocks      m 9   4.03 -> 4.08  m 12  3.96 -> 4.37  m 16  4.3 -> 4.3    m 32  6.2 -> 5.7
+//   K 3072, 64 blocks       m 9   5.8 -> 4.6    m 16  6.9 -> 4.7    (the GEMV's waves do not split it evenly)
+//   K 1024, 192 blocks      m 16  3.95 -> 3.65  m 17  4.09 -> 4.21  m 24  4.33 -> 4.33  m 32  4.1 -> 4.7
+//   K 1024, 256 blocks      m 16  11.2 -> 3.7   m 17  4.29 -> 4.38  m 24  4.18 -> 4.64  m 32  4.4 -> 4.8
+//   K 512, 256 blocks       m 9   3.13 -> 3.26  m 16  3.30 -> 3.27  m 20  3.56 -> 3.76  m 32  3.81 -> 3.81
+// so: never one row; two rows from 1024 blocks on, 3-4 from 512, 5-8 above
+// 256; 9-14 above 256, or where K is more than 4096 or the GEMV splits it
+// unevenly; 15-16 always; 17-32 above 256 or from K 1536 on.
+inline uint32_t W4a16TileBlocks(uint32_t m, uint32_t k, const uint32_t* n, uint32_t count) {
+  uint64_t blocks16 = 0;
+  for (uint32_t i = 0; i < count; ++i) blocks16 += n[i] / 16;
+  if (m < 2 || m > 32) return 0;
+  if (m <= 4 ? blocks16 < (m == 2 ? 1024 : 512) : m <= 8 && blocks16 <= 256) return 0;
+  if (m >= 9 && m <= 14 && blocks16 <= 256 && (k == 512 || k == 2048 || k == 4096)) return 0;
+  if (m >= 17 && blocks16 <= 256 && k <= 1024) return 0;
+  // the tile: as PickTile, x rows whole
+  const double x_bytes = (m <= 16 ? 16.0 : 32.0) * 2.0 * k, w_bytes = 16.0 * (k / 2);
+  uint32_t nb = 0;
+  double best = 0.0;
+  for (uint32_t c : {1u, 2u, 3u, 4u, 6u}) {
+    uint64_t tiles = 0;
+    bool fits = true;
+    for (uint32_t i = 0; i < count; ++i) {
+      fits = fits && n[i] % (16 * c) == 0;
+      tiles += n[i] / (16 * c);
+    }
+    if (!fits) continue;
+    const double rounds = (double)((tiles + kCus - 1) / kCus);
+    const double load = rounds * (x_bytes + c * w_bytes) / 64.0;
+    const double ns = std::max(load, blocks16 * w_bytes / 6200.0) + (rounds - 1.0) * 1500.0 + 0.02 * load;
+    if (!nb || ns < best) {
+      nb = c;
+      best = ns;
+    }
+  }
+  return nb;
+}
+
 }  // namespace pih_amd

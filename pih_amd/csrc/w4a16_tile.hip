@@ -287,52 +287,25 @@ void launch_tile(uint32_t m, uint32_t nb, const W4Params& p, hipStream_t s) {
 
 }  // namespace
 
-// Takes a launch when it is the faster one, else leaves it (`taken` false) to
-// the GEMV kernels.  By measurement (one MI355X, asymmetric, us GEMV -> here;
-// [q, k, v] 384 16-row blocks and o 256 at K 4096, [gate, up] 1536, down 256
-// at K 12288):
-//   m 2   6.4 -> 7.5   4.8 -> 5.9   15.5 -> 13.1   8.9 -> 11.9
-//   m 8   9.8 -> 7.5   5.6 -> 5.9   17.9 -> 13.8   10.9 -> 11.2
-//   m 16  10.4 -> 7.6  6.0 -> 6.0   17.9 -> 13.8   12.9 -> 11.5
-//   m 17  17.2 -> 8.9  9.5 -> 7.0   47.8 -> 16.4   21.3 -> 14.1
-//   m 32  17.6 -> 9.3  9.7 -> 8.1   48.8 -> 16.6   21.6 -> 17.3
-// so: never one row; 2-4 rows from 512 blocks on; 5-8 rows above 256 blocks;
-// 9-32 rows always.
+// Takes a launch when it is the faster one (W4a16TileBlocks), else leaves it
+// (`taken` false) to the GEMV kernels.
 St LaunchW4a16Tile(const W4a16Args* probs, uint32_t count, bool& taken) {
   taken = false;
   const W4a16Args& a0 = probs[0];
-  const uint32_t m = a0.m, k = a0.k, G = k / 128;
-  if (count == 0 || count > kMaxGroup || m < 2 || m > 32 || k % 512 || G > kMaxGroups || 64ull * k > 0xffffffffull) return Ok();
+  const uint32_t m = a0.m, k = a0.k;
+  if (count == 0 || count > kMaxGroup || k % 512 || k / 128 > kMaxGroups || 64ull * k > 0xffffffffull) return Ok();
+  uint32_t n[kMaxGroup];
   uint64_t blocks16 = 0;
   uintptr_t at16 = 0, at4 = 0;
   for (uint32_t i = 0; i < count; ++i) {
-    blocks16 += probs[i].n / 16;
+    n[i] = probs[i].n;
+    blocks16 += n[i] / 16;
     at16 |= reinterpret_cast<uintptr_t>(probs[i].x) | reinterpret_cast<uintptr_t>(probs[i].qweight);
     at4 |= reinterpret_cast<uintptr_t>(probs[i].scales) | reinterpret_cast<uintptr_t>(probs[i].out);
     if (!a0.symmetric) at4 |= reinterpret_cast<uintptr_t>(probs[i].zeros);
   }
   if (at16 % 16 || at4 % 4 || blocks16 > 0x7fffffffull) return Ok();
-  if (m <= 4 ? blocks16 < 512 : m <= 8 ? blocks16 <= 256 : false) return Ok();
-  // the tile: as PickTile of gemm_tile.hip, x rows whole
-  const double x_bytes = (m <= 16 ? 16.0 : 32.0) * 2.0 * k, w_bytes = 16.0 * (k / 2);
-  uint32_t nb = 0;
-  double best = 0.0;
-  for (uint32_t c : {1u, 2u, 3u, 4u, 6u}) {
-    uint64_t tiles = 0;
-    bool fits = true;
-    for (uint32_t i = 0; i < count; ++i) {
-      fits = fits && probs[i].n % (16 * c) == 0;
-      tiles += probs[i].n / (16 * c);
-    }
-    if (!fits) continue;
-    const double rounds = (double)((tiles + kCus - 1) / kCus);
-    const double load = rounds * (x_bytes + c * w_bytes) / 64.0;
-    const double ns = std::max(load, blocks16 * w_bytes / 6200.0) + (rounds - 1.0) * 1500.0 + 0.02 * load;
-    if (!nb || ns < best) {
-      nb = c;
-      best = ns;
-    }
-  }
+  const uint32_t nb = W4a16TileBlocks(m, k, n, count);
   if (!nb) return Ok();
   W4Params p{};
   for (uint32_t i = 0; i < count; ++i) {

@@ -18,4 +18,5 @@ uint32_t bf16_on_tiles(uint32_t m, uint32_t n, uint32_t k, uint32_t f32_out, uin
   return Bf16OnTiles(m, n, k, f32_out != 0, Bf16BigTiles(m, n, k) || Bf16Wide(m, n, k),
                      workspace ? DenseKSplits(m, n, k / 64) : 1, PickTile(true, m, n, 2 * k, 1));
 }
+uint32_t w4a16_blocks(uint32_t m, uint32_t k, const uint32_t* n, uint32_t count) { return W4a16TileBlocks(m, k, n, count); }
 }

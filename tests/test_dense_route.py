@@ -91,3 +91,24 @@ def test_grouped_calls_stay_off_the_128_x_256_tiles(route):
         for n, k in ((1024, 4096), (128, 512), (4096, 8192)):
             for problems in (1, 4, 8, 16):
                 assert route.fp8_on_tiles(m, n, k, problems, 0, 0)
+
+
+def test_w4a16_rule(route):
+    def blocks(m, k, *n):
+        return route.w4a16_blocks(m, k, (ctypes.c_uint32 * len(n))(*n), len(n))
+
+    # Qwen3-8B: [q, k, v], o, [gate, up], down
+    qkv, o, gu, down = (4096, (4096, 1024, 1024)), (4096, (4096,)), (4096, (12288, 12288)), (12288, (4096,))
+    taken = {1: (), 2: (gu,), 4: (gu,), 8: (qkv, gu), 12: (qkv, gu, down), 16: (qkv, o, gu, down),
+             32: (qkv, o, gu, down)}
+    for m, groups in taken.items():
+        for k, n in (qkv, o, gu, down):
+            assert bool(blocks(m, k, *n)) == ((k, n) in groups), (m, k, n)
+    assert blocks(33, 4096, 12288) == 0
+    assert blocks(2, 2048, 6144, 6144) == 0  # 5.54 us on the GEMV, 6.10 on the tiles
+    assert blocks(32, 1024, 3072) == 0 and blocks(32, 1536, 3072)  # 4.1 us on the GEMV, 4.7 on the tiles
+    for m in range(2, 33):
+        for n in ((16,), (48, 96), (16, 32, 4096), (2560,), (9728, 9728)):
+            for k in (512, 1536, 4096, 12288):
+                c = blocks(m, k, *n)
+                assert c in (0, 1, 2, 3, 4, 6) and (not c or all(v % (16 * c) == 0 for v in n))

@@ -74,12 +74,15 @@ def _x(m, k, seed):
 
 # 1, 2, 3, 4 and 6 weight blocks a tile; one K step, fewer steps than stages,
 # many; rows at the edges of the 16- and 32-row operands; k 640 (not a
-# multiple of 512) and 12800 (past the panels) stay on the GEMV
+# multiple of 512), 12800 (past the panels), 2 rows of 512 blocks, 9 and 17
+# rows of few blocks and short K stay on the GEMV
 @pytest.mark.parametrize("sym", [False, True])
 @pytest.mark.parametrize("m,ns,k", [(2, (8192,), 512), (4, (12288, 12288), 1024), (5, (4096, 1024, 1024), 1536),
                                     (9, (48,), 512), (15, (16, 32, 4096), 2560), (16, (12288, 12288), 4096),
                                     (16, (6144,), 12288), (17, (64,), 4096), (31, (9216, 96), 1024),
-                                    (32, (4096, 4096), 2048), (8, (4096,), 640), (20, (256,), 12800)])
+                                    (32, (4096, 4096), 2048), (8, (4096,), 640), (20, (256,), 12800),
+                                    (2, (16384,), 512), (9, (48,), 1536), (14, (4096,), 4096), (15, (4096,), 512),
+                                    (17, (1024,), 1024), (17, (1024,), 1536)])
 def test_exact(eng, m, ns, k, sym):
     import torch
 
