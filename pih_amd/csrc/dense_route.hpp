@@ -115,9 +115,10 @@ inline TilePick PickTile(bool bf16, uint32_t m, uint32_t n, uint32_t row_bytes, 
 // where the walking kernel is MFMA-bound), or what the eight XCDs' L2s must
 // take in where each walks many A rows of few W rows (7 MB/us), the stores
 // (15 KB/us a CU) and a start for each round that is not walked.  The rates
-// are fits to calls within a factor of 2 of each other on both; over 1178
-// calls (M 33-4096, 36 BF16 and 30 FP8 shapes, K 128-28672) the choice was
-// slower than the better kernel by 0.3 % on average, by more than 10 % in 6.
+// are fits to calls within a factor of 2 of each other on both.  Over 1995
+// measured calls (M 1-4096, 41 BF16 shapes with the K split's workspace and
+// without, 30 FP8 shapes, K 128-28672) the choice was 0.2 % slower than the
+// better kernel on average, more than 12 % in 5.
 // Where these tiles were taken always, they lost up to a factor of 2, us 128
 // x 256 tiles -> here: BF16 16384 -> 1024 at M 4096 119 -> 257, 12288 -> 4096
 // at M 1024 103 -> 118, 7680 -> 2560 at M 1024 52 -> 72; FP8 512 -> 32768 at
@@ -131,7 +132,7 @@ inline bool BigTilesFaster(bool bf16, uint32_t m, uint32_t n, uint32_t k, uint32
 
   const uint32_t rows = DenseTileRows(m, n, problems, k_splits);
   const uint64_t big = (uint64_t)((m + rows - 1) / rows) * ((n + 255) / 256) * problems * k_splits;
-  const double step = bf16 ? (rows == 128 ? 0.84 : rows == 64 ? 0.53 : 0.2) : (rows == 128 ? 1.04 : rows == 64 ? 0.79 : 0.62);
+  const double step = bf16 ? (rows == 128 ? 0.84 : rows == 64 ? 0.65 : 0.58) : (rows == 128 ? 1.04 : rows == 64 ? 0.79 : 0.62);
   const double end = (bf16 ? 6.3 : 7.0) * (osz == 2.0 || k_splits > 1 ? 1.0 : 1.4);
   double big_us = std::max(3.0 + rounds(big) * (rb / 128.0 / k_splits * step + end), w_us + 2.0);
   if (k_splits > 1) big_us += 1.7 + (double)k_splits * m * n * 4.0 / 3.3e6;

@@ -76,6 +76,11 @@ BF16_MEASURED = [
     (4096, 512, 7168, 41.2, 66.7), (1024, 2560, 7680, 52.4, 72.0), (256, 4096, 12288, 49.9, 59.4),
     (1024, 4096, 12288, 103.0, 118.3), (200, 8192, 28672, 130.5, 189.7), (128, 5120, 17408, 52.0, 69.2),
     (4096, 4096, 256, 22.3, 36.4), (1000, 5120, 5120, 90.7, 52.4), (2048, 2560, 7680, 125.3, 82.7)]
+# without a workspace: the 128 x 256 tiles unsplit, in 64- and 32-row M tiles
+BF16_NO_WORKSPACE = [
+    (2048, 1024, 4096, 43.1, 29.4), (1024, 1024, 4096, 42.9, 21.0), (301, 4096, 12288, 130.5, 61.9),
+    (512, 4096, 4096, 43.7, 27.7), (1024, 4096, 12288, 134.1, 117.2), (301, 12288, 4096, 52.5, 44.8),
+    (2048, 2048, 6144, 69.5, 61.4), (96, 2048, 6144, 70.8, 16.4)]
 
 
 def test_measured_calls_go_to_the_faster_kernel(route):
@@ -83,6 +88,8 @@ def test_measured_calls_go_to_the_faster_kernel(route):
         assert bool(route.fp8_on_tiles(m, n, k, 1, 0, 1)) == (tiles < other), ("fp8", m, n, k)
     for m, n, k, other, tiles in BF16_MEASURED:
         assert bool(route.bf16_on_tiles(m, n, k, 0, 1)) == (tiles < other), ("bf16", m, n, k)
+    for m, n, k, other, tiles in BF16_NO_WORKSPACE:
+        assert bool(route.bf16_on_tiles(m, n, k, 0, 0)) == (tiles < other), ("bf16 unsplit", m, n, k)
 
 
 def test_grouped_calls_stay_off_the_128_x_256_tiles(route):
