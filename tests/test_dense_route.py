@@ -3,6 +3,8 @@ GEMM runs on and its tile.
 
 * every tile that the rules choose over the shapes of the models here and over
   generic ones is one the kernels are built for;
+* the exact GPU tests of gemm_tile.hip run every tile that is chosen over the
+  models' shapes, with fewer, as many and more K steps than its stages;
 * calls measured on both kernels (one MI355X, us) go to the faster one,
   wherever the two are 5 % apart or more."""
 import ctypes
@@ -56,6 +58,41 @@ def test_only_built_tiles_are_chosen(route, bf16):
                 assert tile in _built(bf16), (m, n, k, problems, tile)
                 # a walked tile has at least 8 K steps; a tile's columns divide n
                 assert n % (16 * tile[1]) == 0 and (not tile[2] or (2 * k if bf16 else k) >= 1024)
+
+
+def _stages(bf16, tile):
+    """LDS stages of a tile and its K steps per 1024 row bytes, as the kernels
+    size them"""
+    mb, nb, grid = tile
+    lds, step = 160 * 1024 - 512, 128 if grid else 256
+    panel = 0 if bf16 else 256 + 16 * mb * 64
+    loads = (mb + nb) * step // 256
+    room = lds - (2 * panel + 4 * 16 * 144 if grid else panel)
+    return min(room // (16 * (mb + nb) * step), 8, 63 // loads + 1), 1024 // step
+
+
+@pytest.mark.parametrize("bf16", [True, False])
+def test_gpu_tests_run_every_tile_of_the_models(route, bf16):
+    import test_gpu_tile as gpu
+
+    used = {}
+    for n, k in QWEN + MLP + HEADS if bf16 else DEEPSEEK:
+        for m in (r for r in ROWS if r <= 2048):
+            taken = route.bf16_on_tiles(m, n, k, 0, 1) if bf16 else route.fp8_on_tiles(m, n, k, 1, 0, 1)
+            if taken:
+                used.setdefault(_tile(route, bf16, m, n, k), (m, n, k))
+    tested = {}
+    for m, n, k in gpu.BF16 + gpu.BF16_TILES if bf16 else gpu.FP8 + gpu.FP8_TILES:
+        if route.bf16_on_tiles(m, n, k, 0, 0) if bf16 else k % 512 == 0 and k <= 8192 and route.fp8_on_tiles(m, n, k, 1, 0, 1):
+            tile = _tile(route, bf16, m, n, k)
+            st, per_kb = _stages(bf16, tile)
+            steps = (2 * k if bf16 else k) * per_kb // 1024
+            tested.setdefault(tile, set()).add((steps > st) - (steps < st))
+    missing = {t: used[t] for t in used if t not in tested}
+    assert not missing, missing
+    for t in used:  # (a walked tile has 8 steps or more and at most 5 stages)
+        assert tested[t] >= ({1} if t[2] else {-1, 1}), (t, tested[t], used[t])
+    assert sum(0 in s for s in tested.values()) >= len(used) // 3
 
 
 # (m, n, k, us on the other kernel, us on the tiles)

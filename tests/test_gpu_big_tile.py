@@ -1,4 +1,8 @@
-"""Dense GEMMs on the MoE kernel's 128 x 256 tiles (large single problems).
+"""Dense GEMMs on the MoE kernel's 128 x 256 tiles (large single problems),
+and beside them the shapes of the same tests that the per-shape tiles of
+gemm_tile.hip take: of the UE8M0 cases K 1152, 1920 and 4224 (no multiples of
+512) and M 2048 of 8192 -> 4096 run on the 128 x 256 tiles, of the BF16 cases
+K 1088 and 1600 (no multiples of 128), all with fp32 scales.
 
 * DeepSeek `launch_fp8_gemm` (UE8M0 scales) and the linear pack's
   `launch_fp8_gemm` (fp32 scales) at shapes whose tile grid fills the GPU:
@@ -71,7 +75,7 @@ def _ue8m0_operands(m, n, k, seed):
     return a, sa, w, sw.reshape(n // 128, k // 128)
 
 
-@pytest.mark.parametrize("m,n,k", [(2048, 4096, 2048), (2048, 4096, 8192), (4096, 2048, 1024)])
+@pytest.mark.parametrize("m,n,k", [(2048, 4096, 2048), (2048, 4096, 8192), (4096, 2048, 1024), (2048, 4096, 1920)])
 def test_deepseek_fp8_gemm_big_tile(eng, m, n, k):
     a, sa, w, sw = _ue8m0_operands(m, n, k, 100 + k)
     got, flag = _ds_fp8(a, sa, w, sw, m, n, k)
@@ -81,8 +85,9 @@ def test_deepseek_fp8_gemm_big_tile(eng, m, n, k):
     assert_close(got[rows], ref, f"big-tile fp8 {m}x{n}x{k}")
 
 
-def test_nan_codes_in_a_and_w(eng):
-    m, n, k = 2048, 4096, 1024
+@pytest.mark.parametrize("k", [1024, 1152])
+def test_nan_codes_in_a_and_w(eng, k):
+    m, n = 2048, 4096
     a, sa, w, sw = _ue8m0_operands(m, n, k, 300)
     a[5, 77] = 0x7F   # NaN code in A (row 5)
     w[1000, 300] = 0xFF  # NaN code in W (column 1000 of every row)
@@ -98,21 +103,23 @@ def test_nan_codes_in_a_and_w(eng):
     assert_close(got[rows], ref, "nan codes as zero")
 
 
-@pytest.mark.parametrize("m,n,k", [(2048, 1024, 4096), (2048, 4096, 1024), (2048, 4096, 384)])
+@pytest.mark.parametrize("m,n,k", [(2048, 1024, 4096), (2048, 4096, 1024), (2048, 1024, 4224), (2048, 4096, 1152),
+                                   (2048, 4096, 384)])
 @pytest.mark.parametrize("where", ["a", "w"])
 def test_nan_code_found_in_tiles(eng, m, n, k, where):
     """One NaN code in A (last M tile, last K block) or in W: the persistent
-    big tiles (32-row M tiles at 2048 x 1024 x 4096) find it in the operand
-    rows of the blocks whose sums it turned into NaN, raise bit 1 only and
-    compute those blocks again with the code as 0.  K = 384 (three K steps)
+    big tiles (K 4224 and 1152; 32-row M tiles at N 1024) find it in the
+    operand rows of the blocks whose sums it turned into NaN, raise bit 1 only
+    and compute those blocks again with the code as 0; the per-shape tiles (K
+    4096 and 1024) do so per element.  K = 384 (three K steps)
     is too short for the persistent tiles: a scan raises the bit, the big
     tiles exit and the checking kernel computes the result."""
     a, sa, w, sw = _ue8m0_operands(m, n, k, 600 + k + (where == "w"))
     a0, w0 = a.copy(), w.copy()
     if where == "a":
-        a[m - 3, k - 5] = 0xFF
+        a[m - 3, k - 5], a0[m - 3, k - 5] = 0xFF, 0
     else:
-        w[n - 7, 1] = 0x7F
+        w[n - 7, 1], w0[n - 7, 1] = 0x7F, 0
     got, flag = _ds_fp8(a, sa, w, sw, m, n, k)
     assert flag == 1, flag
     assert np.isfinite(got).all()
@@ -121,11 +128,12 @@ def test_nan_code_found_in_tiles(eng, m, n, k, where):
     assert_close(got[rows], ref, f"nan code in {where} as zero")
 
 
-def test_nan_code_in_a_skipped_block(eng):
+@pytest.mark.parametrize("k", [4096, 4224])
+def test_nan_code_in_a_skipped_block(eng, k):
     """A NaN code in a 128-k block whose UE8M0 activation scale is 0xFF: the
     reference skips the block before decoding it, so the flag holds bit 2
     only, and that block adds nothing to its row."""
-    m, n, k = 2048, 1024, 4096
+    m, n = 2048, 1024
     a, sa, w, sw = _ue8m0_operands(m, n, k, 650)
     a[100, 1000] = 0x7F
     sa[100, 1000 // 128] = 0xFF
@@ -140,7 +148,8 @@ def test_nan_code_in_a_skipped_block(eng):
     assert_close(got[rows], ref, "code in a skipped block")
 
 
-def test_nan_code_with_overflow_elsewhere(eng):
+@pytest.mark.parametrize("k", [4096, 4224])
+def test_nan_code_with_overflow_elsewhere(eng, k):
     """A NaN code in A row 7 and, in other columns, sums that overflow: bit 1
     from the code and bit 4 from the overflow (the overflowing elements are
     left unwritten, as the reference does, row 7's among them); the other
@@ -149,7 +158,7 @@ def test_nan_code_with_overflow_elsewhere(eng):
 
     from pih_amd.device import ptr, stream_handle
 
-    m, n, k = 2048, 1024, 4096
+    m, n = 2048, 1024
     a = np.zeros((m, k), np.uint8)
     a[:, :128] = 0x7E  # 448
     w = np.zeros((n, k), np.uint8)
@@ -211,10 +220,11 @@ def test_linear_fp8_gemm_nan_code_f32_scales(eng, out_type):
     assert_close(got[rows], ref, "f32-scale nan code as zero")
 
 
-def test_code_bit_already_set(eng):
+@pytest.mark.parametrize("k", [1024, 1152])
+def test_code_bit_already_set(eng, k):
     """A flag that already holds bit 1 (a poisoned lane) before the call:
     the bit stays, and the result is the same."""
-    m, n, k = 2048, 4096, 1024
+    m, n = 2048, 4096
     a, sa, w, sw = _ue8m0_operands(m, n, k, 400)
     clean, flag0 = _ds_fp8(a, sa, w, sw, m, n, k)
     assert flag0 == 0
@@ -256,7 +266,8 @@ def test_linear_fp8_gemm_big_tile_f32_scales(eng, out_type):
     assert_close(got[rows], ref, f"big-tile fp8 f32-scale out {out_type}")
 
 
-@pytest.mark.parametrize("m,n,k,out_type", [(1024, 8192, 1024, 1), (2048, 4096, 1536, 2)])
+@pytest.mark.parametrize("m,n,k,out_type", [(1024, 8192, 1024, 1), (2048, 4096, 1536, 2), (1024, 8192, 1088, 1),
+                                            (2048, 4096, 1600, 2)])
 def test_bf16_gemm_big_tile(eng, m, n, k, out_type):
     import torch
 
@@ -279,17 +290,19 @@ def test_bf16_gemm_big_tile(eng, m, n, k, out_type):
     assert_close(got[rows], ref, f"big-tile bf16 {m}x{n}x{k}")
 
 
-@pytest.mark.parametrize("m,n,k", [(2048, 1024, 4096), (1000, 2048, 4096), (2048, 1280, 4608), (128, 4096, 12288),
-                                   (96, 1024, 4096)])
+@pytest.mark.parametrize("m,n,k,split", [(2048, 1024, 4096, False), (1000, 2048, 4096, False), (2048, 1280, 4608, True),
+                                         (128, 4096, 12288, True), (96, 1024, 4096, False), (2048, 1024, 4160, True),
+                                         (96, 1024, 4160, True), (1000, 2560, 7680, True), (2048, 256, 16384, True)])
 @pytest.mark.parametrize("out_type", [abi.OUTPUT_BF16, abi.OUTPUT_F32])
-def test_bf16_gemm_k_split(eng, m, n, k, out_type):
+def test_bf16_gemm_k_split(eng, m, n, k, split, out_type):
     """launch_bf16_gemm with the queried workspace at shapes with fewer big
-    tiles than CUs (the Qwen3-8B k/v projections at M 2048: 4 K splits; M
-    1000: a partial M tile; 4608 -> 1280: 3 splits; batches of 96 and 128
-    rows: 8 splits, one partial M tile; without the workspace they run
-    unsplit on 32-row M tiles): the fp32 partial sums go to the
-    workspace (filled with NaN bytes first, so an element no split writes
-    would show) and are summed in split order.  Sampled rows against the
+    tiles than CUs.  `split`: K is split on the 128 x 256 tiles (4608 -> 1280
+    and 7680 -> 2560 at M 1000, a partial M tile: 3 and 3 splits; 4160 -> 1024:
+    5; 16384 -> 256 and batches of 96 and 128 rows: up to 8), the fp32
+    partial sums go to the workspace (filled with NaN bytes first, so an
+    element no split writes would show) and are summed in split order; the
+    other shapes run on the per-shape tiles and leave it alone, as all do
+    without a workspace where K is a multiple of 128.  Sampled rows against the
     oracle, every row's sum against a float64 checksum, and the whole output
     against the unsplit launch (workspace 0) within the fp32 reordering of
     the K sum (bf16: one unit in the last place)."""
@@ -320,39 +333,44 @@ def test_bf16_gemm_k_split(eng, m, n, k, out_type):
         host = to_host(out)
         return oracle.bf16_bits_to_f32(host) if out_type == abi.OUTPUT_BF16 else host
 
-    split, whole = run(True), run(False)
-    assert np.all(np.isfinite(split))
+    whole = run(False)
+    assert bool((ws == 0xFF).all())
+    got = run(True)
+    assert bool((ws != 0xFF).any()) == split
+    assert np.all(np.isfinite(got))
     rows = np.unique(np.concatenate([np.linspace(0, m - 1, 24).astype(np.int64), [127, 128, m - 1]]))
     rows = rows[rows < m]
     ref = oracle.bf16_gemm(np.ascontiguousarray(x[rows]), w)
-    assert_close(split[rows], ref, f"k-split bf16 {m}x{n}x{k}")
+    assert_close(got[rows], ref, f"k-split bf16 {m}x{n}x{k}")
     colsum = oracle.bf16_bits_to_f32(w).astype(np.float64).sum(axis=0)
     want = oracle.bf16_bits_to_f32(x).astype(np.float64) @ colsum
-    have = split.astype(np.float64).sum(axis=1)
-    bound = np.abs(split).astype(np.float64).sum(axis=1) * 2.0 ** -8 + 1e-3
+    have = got.astype(np.float64).sum(axis=1)
+    bound = np.abs(got).astype(np.float64).sum(axis=1) * 2.0 ** -8 + 1e-3
     assert np.all(np.abs(have - want) <= bound), "k-split row checksums"
     if out_type == abi.OUTPUT_F32:
         # fp32 sums of the same products in two orders (outputs ~1.3 rms)
-        assert np.all(np.abs(split - whole) <= 2e-5 + np.abs(whole) * 1e-5)
+        assert np.all(np.abs(got - whole) <= 2e-5 + np.abs(whole) * 1e-5)
     else:
         # one bf16 rounding each of two fp32 sums that differ in the order of
         # their K parts (~1e-6 here): one unit in the last place, plus slack
         # for results that cancel to near zero
-        ulp = np.maximum(np.abs(whole), np.abs(split)) * 2.0 ** -7 + 1e-4
-        assert np.all(np.abs(split - whole) <= ulp)
+        ulp = np.maximum(np.abs(whole), np.abs(got)) * 2.0 ** -7 + 1e-4
+        assert np.all(np.abs(got - whole) <= ulp)
 
 
-def test_big_tile_nonfinite_results_skipped(eng):
+@pytest.mark.parametrize("k", [1024, 1152])
+def test_big_tile_nonfinite_results_skipped(eng, k):
     """Sums that overflow (UE8M0 weight scale 2^127 on one 128-row block)
     raise bit 4 and leave their elements unwritten, as the reference's
     fp8_gemm_kernel skips them (deepseek_fp8_gemm.cu:67-70); the other
-    columns hold the oracle's values.  M = 2048 runs the persistent big-tile
-    kernel, whose waves with such an element store per element."""
+    columns hold the oracle's values.  K 1152 runs the persistent big-tile
+    kernel, whose waves with such an element store per element, K 1024 the
+    tile-walking one, which does so too."""
     import torch
 
     from pih_amd.device import ptr, stream_handle
 
-    m, n, k = 2048, 4096, 1024
+    m, n = 2048, 4096
     a = np.zeros((m, k), np.uint8)
     a[:, :128] = 0x7E  # 448
     w = np.zeros((n, k), np.uint8)

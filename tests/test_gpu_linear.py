@@ -98,15 +98,28 @@ def test_bf16_gemv_decode(eng, m, n, k):
 @pytest.mark.parametrize("m,n,k", [(5, 1024, 4096), (20, 1024, 4096), (40, 256, 1024), (64, 8192, 1024),
                                    (16, 8192, 1024), (64, 1024, 4096), (24, 256, 1152)])
 def test_bf16_gemv_mid_m(eng, m, n, k):
-    """4 < M <= 64: every configuration of the line-loading mid-M kernel
-    (M tiles 1-4; 8192 rows take the 4-W-block and 4-wave variants) and, at
-    K = 1152 (36 steps, no even split over 8 waves with 4-step batches),
-    the gemv_kernel fallback."""
+    """4 < M <= 64, once on 16-byte boundaries (most of them on the per-shape
+    tiles) and once with W 8 bytes off, which only the GEMV takes: every
+    configuration of the line-loading mid-M kernel (M tiles 1-4; 8192 rows
+    take the 4-W-block and 4-wave variants) and, at K = 1152 (36 steps, no
+    even split over 8 waves with 4-step batches), the gemv_kernel fallback."""
+    import torch
+
+    from pih_amd.linear import bf16_gemm
+
     a = synth.bf16_normal(synth.config_seed(2, 60 + m), (m, k))
     w = synth.bf16_normal(synth.config_seed(2, 70 + n), (n, k), std=0.02)
     ref = oracle.bf16_gemm(a, w)
     assert_close(_bf16_gemm(a, w, abi.OUTPUT_BF16), ref, f"bf16 gemv {m}x{n}x{k}")
     assert_close(_bf16_gemm(a, w, abi.OUTPUT_F32, use_ws=False), ref, f"bf16 gemv no-ws {m}x{n}x{k}")
+    ad, wd = (to_dev(v).view(torch.bfloat16) for v in (a, w))
+    off = torch.empty(n * k + 8, dtype=torch.bfloat16, device="cuda")[4:4 + n * k].view(n, k)
+    off.copy_(wd)
+    assert off.data_ptr() % 16 == 8
+    for out_type in (abi.OUTPUT_BF16, abi.OUTPUT_F32):
+        got = bf16_gemm(ad, off, out_type)
+        _sync()
+        assert_close(got.float().cpu().numpy(), ref, f"bf16 gemv, W off, {m}x{n}x{k}")
 
 
 # ----------------------------------------------------------------- W4A16
@@ -162,10 +175,13 @@ def test_w4a16_asym(eng, m, n, k):
 
 
 @pytest.mark.parametrize("m,n,k", [(5, 1024, 4096), (20, 1024, 4096), (32, 8192, 1024), (9, 8192, 1024),
-                                   (9, 256, 1152)])
+                                   (9, 256, 1152), (14, 4096, 2048), (20, 1024, 1024), (32, 4096, 1024),
+                                   (5, 8192, 13312), (5, 16384, 13312)])
 def test_w4a16_asym_mid_m(eng, m, n, k):
-    """4 < M <= 32 on the mid-M kernel (one and two M tiles, 8 and 4 waves);
-    K = 1152 (9 groups) does not split over its waves and takes
+    """4 < M <= 32: the mid-M kernel with one M tile (M 5 and 14 of 256 blocks
+    and fewer), two (K 1024) and 2 and 4 W blocks a wave (K 13312, past the
+    tiles' scale panels); M 20 and 32 otherwise and 8192 rows run on the
+    tiles; K = 1152 (9 groups) does not split over its waves and takes
     gemv_kernel."""
     q, s, z = synth.int4_asym_weight(synth.config_seed(3, 4000 + n + k), n, k)
     x = synth.bf16_normal(synth.config_seed(3, 4100 + m), (m, k))
@@ -175,11 +191,12 @@ def test_w4a16_asym_mid_m(eng, m, n, k):
     assert_close(oracle.bf16_bits_to_f32(got), oracle.bf16_bits_to_f32(ref), f"w4a16 asym {m}x{n}x{k}")
 
 
-@pytest.mark.parametrize("m", [9, 20])
-def test_w4a16_symmetric_mid_m_and_errors(eng, m):
-    """Reference format on the mid-M kernel: results against the oracle, then
-    a reserved nibble raises code 12 and a negative scale code 13."""
-    n, k = 1024, 2048
+@pytest.mark.parametrize("m,k", [(9, 2048), (20, 2048), (20, 1024)])
+def test_w4a16_symmetric_mid_m_and_errors(eng, m, k):
+    """Reference format on the mid-M kernel (M 9, and M 20 of K 1024) and on
+    the tiles: results against the oracle, then a reserved nibble raises code
+    12 and a negative scale code 13."""
+    n = 1024
     q, s = synth.int4_sym_weight(synth.config_seed(3, 4200 + m), n, k)
     x = synth.bf16_normal(synth.config_seed(3, 4300 + m), (m, k))
     got, flag = _w4a16(x, q, s, None, abi.W4A16_SYMMETRIC, m, n, k)
@@ -190,7 +207,7 @@ def test_w4a16_symmetric_mid_m_and_errors(eng, m):
     _, flag = _w4a16(x, q2, s, None, abi.W4A16_SYMMETRIC, m, n, k)
     assert flag == 12
     s2 = s.copy()
-    s2[1000, 15] = 0xBC00  # -1.0
+    s2[1000, k // 128 - 1] = 0xBC00  # -1.0
     _, flag = _w4a16(x, q, s2, None, abi.W4A16_SYMMETRIC, m, n, k)
     assert flag == 13
 
@@ -223,8 +240,9 @@ def _w4a16_grouped(xs, weights, fmt, m, k):
 @pytest.mark.parametrize("m", [1, 4, 16])
 def test_w4a16_grouped_qkv_and_gate_up(eng, m):
     """q/k/v and gate/up of Qwen3-8B as two grouped launches (one input per
-    problem); each output against the oracle's strict-k sum.  m = 1 and 4
-    run the small-M kernel, m = 16 the mid-M kernel, one launch per group."""
+    problem); each output against the oracle's strict-k sum.  m = 1 and
+    [q, k, v] at m = 4 run the GEMV's small-M kernel, the others the tiles, one
+    launch per group."""
     k = 4096
     for ns in ((4096, 1024, 1024), (12288, 12288)):
         weights = [synth.int4_asym_weight(synth.config_seed(3, 3000 + i + n), n, k) + (n,) for i, n in enumerate(ns)]

@@ -1,4 +1,6 @@
-"""GPU parity of the small-M GEMM path (gemm_small_m.hip): the dense FP8
+"""GPU parity of the small-M GEMM path (gemm_small_m.hip; UE8M0 scales: at
+K 640, 1152, 4224, 7296 and 12288, which the tiles of gemm_tile.hip do not take,
+and up to 8 rows of 1024 -> 256; the other K run on those): the dense FP8
 GEMM (UE8M0 through the DeepSeek table, fp32 scales through the linear
 pack), the FP4 x FP8 GEMM and the grouped FP8 GEMM with at most 64
 activation rows, and with up to 256 rows in 64-row chunks where the
@@ -78,7 +80,8 @@ def _fp8_inputs(seed, m, n, k):
 
 
 @pytest.mark.parametrize("m", [1, 5, 16, 17, 33, 64, 65, 128, 200])
-@pytest.mark.parametrize("n,k", [(1024, 4096), (384, 7168), (256, 1024), (128, 12288)])
+@pytest.mark.parametrize("n,k", [(1024, 4096), (384, 7168), (256, 1024), (128, 12288), (1024, 4224), (384, 7296),
+                                 (256, 1152)])
 def test_fp8_ue8m0_small_m(eng, m, n, k):
     a, sa, w, sw = _fp8_inputs(synth.config_seed(4, 15000 + m + n), m, n, k)
     got, flag = _ds_fp8(a, sa, w, sw)
@@ -154,15 +157,15 @@ def test_small_m_error_bits(eng):
 
 
 @pytest.mark.parametrize("t", [1, 3, 16, 100])
-def test_grouped_fp8_small_t(eng, t):
-    """The attention wo_a geometry (G = 8, 1024, 4096) at decode token
-    counts (and at 100, two row chunks): A row t * 8 + g of the quantised
-    input feeds group g."""
+@pytest.mark.parametrize("g,ng,kg", [(8, 1024, 4096), (4, 256, 640)])
+def test_grouped_fp8_small_t(eng, t, g, ng, kg):
+    """The attention wo_a geometry (G = 8, 1024, 4096; on the per-shape tiles)
+    and K 640 (the small-M kernel) at decode token counts (and at 100, two row
+    chunks): A row t * G + g of the quantised input feeds group g."""
     import torch
 
     from pih_amd.device import ptr, stream_handle
 
-    g, ng, kg = 8, 1024, 4096
     x = synth.bf16_normal(synth.config_seed(4, 15400 + t), (t * g, kg))
     w = _codes(synth.config_seed(4, 15401), (g * ng, kg))
     sw = (112 + synth.splitmix64(15402, g * (ng // 128) * (kg // 128)) % np.uint64(6)).astype(np.uint8)

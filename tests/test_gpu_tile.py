@@ -33,16 +33,29 @@ def _ints(shape, seed, high=3):
     return torch.randint(-high, high + 1, shape, device="cuda", generator=g).float()
 
 
-# m, n, k around: one and two rows, whole and ragged 16-row blocks, 1-5
-# blocks a tile, 48-column tiles (n / 16 not even), fewer K steps than LDS
-# stages (k 128: one step), several rounds, the tile-walking kernel (128 x
-# 128, 192 x 128 and 256 x 128 tiles, more tiles than CUs and fewer)
+# m, n, k around: two rows, whole and ragged 16-row blocks, n / 16 not even,
+# one K step (k 128), several rounds, the tile-walking kernel (128 x 128, 192 x
+# 128 and 256 x 128 tiles, more tiles than CUs and fewer), and calls that stay
+# on the GEMV, the 128 x 256 and the 128 x 128 kernel
 BF16 = [(2, 16, 128), (3, 64, 256), (16, 1024, 384), (17, 4096, 128), (33, 48, 1152), (48, 768, 512),
         (57, 12288, 512), (64, 1024, 4096), (65, 256, 640), (80, 4096, 256), (127, 512, 1024), (200, 12288, 512),
         (301, 1024, 2048), (600, 9216, 512), (1000, 4096, 1024), (2048, 4096, 512), (2047, 12288, 512)]
+# every tile that the Qwen3 projections, MLP blocks and LM heads get, with a
+# ragged last tile and fewer, as many and more K steps than its LDS stages
+# (test_dense_route.py checks that none is left out)
+BF16_TILES = [
+    (2, 16, 256), (2, 16, 1024), (2, 16, 1152), (2, 5120, 256), (2, 5120, 1024), (2, 5120, 1152), (33, 1536, 128),
+    (17, 2560, 1024), (17, 2560, 1152), (33, 3072, 128), (17, 5120, 1024), (17, 5120, 1152), (97, 3072, 128),
+    (17, 9216, 1024), (33, 5120, 128), (33, 5120, 1024), (33, 9216, 128), (33, 9216, 768), (33, 9216, 1024),
+    (193, 2560, 128), (193, 2560, 640), (193, 2560, 768), (49, 5120, 128), (49, 5120, 768), (49, 5120, 1024),
+    (49, 9216, 128), (49, 9216, 640), (49, 9216, 768), (600, 1280, 128), (600, 1280, 512), (600, 1280, 640),
+    (150, 9216, 128), (150, 9216, 384), (150, 9216, 512), (65, 9216, 128), (65, 9216, 512), (65, 9216, 640),
+    (193, 5120, 128), (193, 5120, 512), (193, 5120, 640), (81, 9216, 128), (81, 9216, 512), (81, 9216, 640),
+    (1000, 1280, 128), (1000, 1280, 384), (1000, 1280, 512), (97, 9216, 128), (97, 9216, 384), (97, 9216, 512),
+    (600, 2560, 128), (600, 2560, 384), (600, 2560, 512), (129, 12288, 512), (257, 12288, 512), (390, 12288, 512)]
 
 
-@pytest.mark.parametrize("m,n,k", BF16)
+@pytest.mark.parametrize("m,n,k", BF16 + BF16_TILES)
 def test_bf16_exact(eng, m, n, k):
     import torch
 
@@ -154,14 +167,23 @@ def _run_fp8(a, sa, w, sw, out_type):
     return out, int(flag.item())
 
 
-# k 8192 is the deepest scale panel; k 512 and 1024 have fewer steps than
-# stages; 768 (not a multiple of 512) and 8704 (deeper) stay on other kernels
+# k 8192 is the deepest scale panel; 768 (not a multiple of 512) and 8704
+# (deeper), and some of the smallest calls, stay on other kernels
 FP8 = [(1, 128, 512), (3, 1024, 1024), (4, 4096, 8192), (16, 2048, 512), (17, 128, 1536), (40, 256, 768),
        (50, 4096, 512), (75, 1024, 2048), (129, 4096, 1024), (33, 128, 8704), (301, 2048, 1024), (301, 32768, 1024),
        (700, 4096, 2048), (2048, 1024, 1024), (2047, 8192, 1024)]
+# every tile that the DeepSeek projections get, as BF16_TILES
+FP8_TILES = [
+    (2, 128, 1536), (2, 128, 2048), (2, 128, 2560), (2, 32768, 512), (2, 32768, 1024), (2, 32768, 1536),
+    (17, 2560, 512), (17, 2560, 2048), (17, 2560, 2560), (17, 5120, 512), (17, 5120, 2048), (17, 5120, 2560),
+    (17, 32768, 512), (17, 32768, 1024), (33, 5120, 512), (33, 5120, 2048), (33, 9216, 512), (33, 9216, 1536),
+    (97, 9216, 512), (97, 9216, 1024), (49, 5120, 512), (49, 5120, 1536), (49, 5120, 2048), (49, 9216, 512),
+    (49, 9216, 1024), (49, 9216, 1536), (150, 9216, 512), (150, 9216, 1024), (65, 9216, 512), (65, 9216, 1024),
+    (65, 9216, 1536), (81, 9216, 512), (81, 9216, 1024), (97, 12288, 512), (97, 12288, 1024), (129, 12288, 1024),
+    (257, 12288, 1024)]
 
 
-@pytest.mark.parametrize("m,n,k", FP8)
+@pytest.mark.parametrize("m,n,k", FP8 + FP8_TILES)
 def test_fp8_exact(eng, m, n, k):
     import torch
 
@@ -173,7 +195,7 @@ def test_fp8_exact(eng, m, n, k):
         assert torch.equal(got, ref.float().bfloat16() if out_type == 1 else ref.float())
 
 
-@pytest.mark.parametrize("m,n,k", [(20, 256, 1024), (301, 2048, 1024), (700, 8192, 1024)])
+@pytest.mark.parametrize("m,n,k", [(20, 256, 1024), (301, 2048, 1024), (301, 4096, 1024), (700, 8192, 1024)])
 def test_fp8_codes_and_invalid_scales(eng, m, n, k):
     """NaN codes count as 0 and raise bit 1, 0xFF scales leave their block out
     and raise bit 2, in one-tile-per-block and in walked tiles; a code in a
