@@ -66,12 +66,12 @@ struct TilePick {
 };
 
 // The tile for a shape, by an estimate of its time: the rounds of tiles on the
-// CUs times what a CU loads for one (at the ~64 GB/s it takes in while part of
-// its lines come from HBM), no less than the weights at the 6.2 TB/s they
-// stream at, and 1.5 us for each round after the first (the start-up that the
-// tile-walking kernel hides).  16 x 16 tiles share a CU two at a time: their
-// weights were measured to stream at 7 TB/s (12288 x 4096 bf16 at m 8: 16.5
-// us, 18.4 with 16 x 48 tiles) and a round is 512 of them, 1.1 us apart.
+// CUs times what a CU loads for one (at ~64 GB/s), no less than the weights at
+// the 6.2 TB/s they stream at, and 1.5 us for each round after the first (the
+// start-up that the tile-walking kernel hides).  16 x 16 tiles share a CU two
+// at a time: their weights were measured to stream at 7 TB/s (12288 x 4096
+// bf16 at m 8: 16.5 us, 18.4 with 16 x 48 tiles) and a round is 512 of them,
+// 1.1 us apart.
 inline TilePick PickTile(bool bf16, uint32_t m, uint32_t n, uint32_t row_bytes, uint32_t problems) {
   TilePick best;
   double best_ns = 0.0;

@@ -1099,8 +1099,10 @@ St LaunchMx32Gemm(const Mx32GemmArgs& a) {
 
 uint64_t Bf16GemmWorkspaceBytes(uint32_t m, uint32_t n, uint32_t k) {
   if (m <= 64) return Bf16GemvWorkspaceBytes(m, n, k);
-  // the big tiles' K split (fp32 partial sums); without this workspace the
-  // call runs unsplit
+  // the big tiles' K split (fp32 partial sums), for the calls that the
+  // per-shape tiles leave to them (Bf16OnTiles; K % 128 == 64 or operands off
+  // 16-byte boundaries, which the query does not see); without this workspace
+  // such a call runs unsplit
   if (n % 128 || k % 64 || !Bf16BigTiles(m, n, k)) return 0;
   const uint32_t splits = DenseKSplits(m, n, k / 64);
   return splits > 1 ? (uint64_t)splits * m * n * 4 : 0;

@@ -3,30 +3,29 @@
 // 128 k, one per 128 W rows and 128 k), fp32 accumulation.
 //
 // What bounds such a call: not HBM alone.  A block reads its A rows as well as
-// its W rows, and a CU takes in ~64 GB/s while part of its lines come from HBM
-// or the MALL (~100 GB/s when all hit L2; deeper rings, other row patterns,
-// staggered K orders and an L2 prefetch through the scalar cache did not raise
-// it), against the ~23 GB/s that is its share of HBM.  So a tile of TM x TN
-// costs a CU (TM + TN) x row bytes at that rate, and what matters is that all
-// 256 CUs have a tile and that TM + TN is no larger than that takes.  The
-// 128 x 256 tiles of gemm_fp8_moe.hip leave most CUs idle at these sizes, and
-// the 16-row GEMV blocks read all of A for every 16 weight rows in the waves'
-// own loads.  Here the tile is chosen per call (PickTile) from 16-row steps
-// both ways.  Figures: at the dispatch rules in gemm_mfma.hip.
+// its W rows, and a CU takes in ~64 GB/s (55-65, fitted to the measured times
+// of calls of one round, where the tiles' row bytes are known), against the
+// ~23 GB/s that is its share of HBM.  So a tile of TM x TN costs a CU (TM + TN)
+// x row bytes at that rate, and what matters is that all 256 CUs have a tile
+// and that TM + TN is no larger than that takes.  The 128 x 256 tiles of
+// gemm_fp8_moe.hip leave most CUs idle at these sizes, and the 16-row GEMV
+// blocks read all of A for every 16 weight rows in the waves' own loads.  Here
+// the tile is chosen per call (PickTile) from 16-row steps both ways.  Which
+// calls run here, and both sides' times: dense_route.hpp, gemm_mfma.hip.
 //
 // A block is 4 multiplying and 4 loading waves: a wave issues in order, and a
 // DMA that the full load queue does not take yet would hold back the MFMAs
 // behind it (one kind of wave doing both: 5-15 % slower).  A K step is 256
 // bytes of every tile row, moved into LDS by DMA (global_load_lds_dwordx4, 4
 // rows x 256 bytes an instruction, the same number from every loading wave),
-// kStages steps deep: one wait and one barrier a step.  16-byte chunk c of row r sits in slot c ^ (r & 15) of its 256
-// bytes, so that a fragment read (16 rows, one chunk each) covers the 64
-// banks once.  The multiplying waves split the step's K, not the tile: each reads its
-// share of every row, so an LDS byte is read once (bf16: four k quarters;
-// e4m3: two 128-k halves, times two halves of the W rows), and the waves'
-// sums meet in LDS at the end in a fixed order, from which whole output rows
-// are stored.  The MFMA's first operand is W, so a lane's four results are
-// four consecutive columns of one row.
+// kStages steps deep: one wait and one barrier a step.  16-byte chunk c of row
+// r sits in slot c ^ (r & 15) of its 256 bytes, so that a fragment read (16
+// rows, one chunk each) covers the 64 banks once.  The multiplying waves split
+// the step's K, not the tile: each reads its share of every row, so an LDS
+// byte is read once (bf16: four k quarters; e4m3: two 128-k halves, times two
+// halves of the W rows), and the waves' sums meet in LDS at the end in a fixed
+// order, from which whole output rows are stored.  The MFMA's first operand is
+// W, so a lane's four results are four consecutive columns of one row.
 //
 // e4m3 NaN codes count as 0 and raise the code bit, as the reference decodes
 // them (plugins/kernels/deepseek-v4-sm89/native/deepseek_fp8_gemm.cu:11-70):

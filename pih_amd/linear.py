@@ -46,7 +46,7 @@ def route_plan_workspace(tokens: int, topk: int, experts: int) -> int:
 
 def bf16_gemm_workspace(m: int, n: int, k: int) -> int:
     """Scratch bytes launch_bf16_gemm can use at this shape (query_workspace;
-    0: none)."""
+    0: none).  A call that runs on the per-shape tiles leaves them alone."""
     out = (abi.C.c_uint64 * 1)()
     q = abi.request(abi.LN["workspace_query"], kind=abi.WORKSPACE_BF16_GEMM, m=m, n=n, k=k,
                     bytes_u64=abi.C.addressof(out))
@@ -278,7 +278,8 @@ class QwenLmHead:
     bank of GemmPlans for 1..maximum_rows rows (at most 32) over the tied
     [151936, 1024] bf16 weight with fp32 logits; ``execute`` rejects a row
     count outside the bank.  Here every row count is the same
-    ``launch_bf16_gemm`` call (the weight-streaming GEMV, no workspace)."""
+    ``launch_bf16_gemm`` call (one row the weight-streaming GEMV, more the 128 x
+    256 tiles; no workspace)."""
 
     def __init__(self, maximum_rows: int):
         if not 1 <= maximum_rows <= 32:
