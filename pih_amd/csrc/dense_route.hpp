@@ -200,16 +200,17 @@ inline bool Bf16Wide(uint32_t m, uint32_t n, uint32_t k) {
 // groups, as the other kernels take them there).  Left out: very wide weights
 // up to 128 rows (HBM-bound on the 128 x 256 tiles: 6.1 TB/s; 129 rows 270 ->
 // 242 us here); what the GEMV's blocks have done before these have started, 5
-// to 16 rows of K 1024 (which its waves split evenly) and N <= 4096, of N <=
-// 256 and K <= 768, of N <= 1024 and K <= 256, and up to 32 of K 128 (us GEMV
-// -> here: 1024 -> 1024 at M 8 3.35 -> 3.55, 1024 -> 3072 at M 16 3.85 -> 4.05,
-// 512 -> 256 at M 8 2.5 -> 3.0, 256 -> 1024 at M 8 2.45 -> 2.9, 128 -> 1024 at M
-// 8 2.1 -> 2.8; but 768 -> 1024 at M 8 3.7 -> 3.1, 1152 -> 256 at M 8 4.0 ->
-// 3.6); and what the 128 x 256 tiles are faster for.
+// to 16 rows of N <= 256 and K <= 768 or of N <= 1024 and K <= 256, and up to 32
+// of K 128 (us GEMV -> here: 512 -> 256 at M 8 2.5 -> 3.0, 256 -> 1024 at M 8
+// 2.45 -> 2.9, 128 -> 1024 at M 8 2.1 -> 2.8; but 768 -> 1024 at M 8 3.7 -> 3.1,
+// 1152 -> 256 at M 8 4.0 -> 3.6); and what the 128 x 256 tiles are faster for.
+// (K 1024, which the GEMV's waves split evenly: alone and with cold weights 1024
+// -> 3072 at M 16 3.85 -> 4.05, but the MLP block of two such calls, SiLU and
+// 3072 -> 1024 18.5 -> 17.6.)
 inline bool Bf16OnTiles(uint32_t m, uint32_t n, uint32_t k, bool f32_out, bool big, uint32_t k_splits,
                         const TilePick& t) {
   if (m < 2 || (m > 64 && n % 128) || (m <= 128 && Bf16Wide(m, n, k))) return false;
-  const bool short_k = (k == 1024 && n <= 4096) || (k <= 768 && n <= 256) || (k <= 256 && n <= 1024);
+  const bool short_k = (k <= 768 && n <= 256) || (k <= 256 && n <= 1024);
   if ((m >= 5 && m <= 16 && short_k) || (m <= 32 && k == 128)) return false;
   return m <= 64 || !big || !BigTilesFaster(true, m, n, k, 1, f32_out, t, k_splits);
 }

@@ -105,8 +105,7 @@ FP8_MEASURED = [
     (2048, 4096, 6144, 60.1, 64.9), (4096, 8192, 8192, 284.6, 309.6), (2048, 12288, 4096, 121.6, 128.5),
     (512, 4096, 8192, 50.5, 29.3), (1024, 2048, 7168, 47.5, 26.0), (2048, 32768, 1024, 127.0, 101.0)]
 BF16_MEASURED = [
-    (8, 1024, 128, 2.08, 2.77), (8, 1024, 1024, 3.35, 3.55), (16, 3072, 1024, 3.85, 4.05), (8, 256, 512, 2.5, 3.0),
-    (8, 1024, 768, 3.7, 3.1), (2, 12288, 4096, 20.3, 17.7),
+    (8, 1024, 128, 2.08, 2.77), (8, 256, 512, 2.5, 3.0), (8, 1024, 768, 3.7, 3.1), (2, 12288, 4096, 20.3, 17.7),
     (17, 12288, 4096, 21.6, 18.7), (57, 1024, 4096, 11.0, 6.4), (200, 4096, 4096, 25.0, 17.3),
     (200, 28672, 4096, 87.0, 78.0), (2048, 12288, 4096, 183.0, 163.0), (2048, 4096, 12288, 175.0, 160.0),
     (4096, 1024, 16384, 119.4, 257.1), (2048, 1024, 16384, 68.9, 121.5), (2048, 256, 16384, 42.5, 77.0),
