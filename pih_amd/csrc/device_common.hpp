@@ -221,6 +221,46 @@ __device__ __forceinline__ float ue8m0_value(uint32_t b) {
   return b == 0 ? 0x1p-127f : __uint_as_float(b << 23);
 }
 
+// non-zero when any byte of w is 0xFF
+__device__ __forceinline__ uint32_t ff_bytes(uint32_t w) {
+  const uint32_t n = ~w;
+  return (n - 0x01010101u) & ~n & 0x80808080u;
+}
+
+// 8 nibbles of one word (nibble j = k offset j) -> eight bf16 values
+// 128 + u_j in the order k = 0, 2, 4, 6, 1, 3, 5, 7: the low nibbles of the
+// four bytes are the even k, the high nibbles the odd k, and one v_perm per
+// pair places two of them under the 0x43 exponent byte of 128.  x takes the
+// same order (x_in_nibble_order), so the MFMA sees matching k on both
+// operands.
+__device__ __forceinline__ v4i nibbles_to_bf16(uint32_t w) {
+  const uint32_t lo = w & 0x0F0F0F0Fu, hi = (w >> 4) & 0x0F0F0F0Fu;
+  constexpr uint32_t kExp = 0x43434343u;
+  return v4i{(int)__builtin_amdgcn_perm(kExp, lo, 0x04010400u),   // k0, k2
+             (int)__builtin_amdgcn_perm(kExp, lo, 0x04030402u),   // k4, k6
+             (int)__builtin_amdgcn_perm(kExp, hi, 0x04010400u),   // k1, k3
+             (int)__builtin_amdgcn_perm(kExp, hi, 0x04030402u)};  // k5, k7
+}
+// Eight bf16 x values (k = 0..7) into the order nibbles_to_bf16 produces.
+__device__ __forceinline__ v4i x_in_nibble_order(v4i v) {
+  const uint32_t w0 = (uint32_t)v[0], w1 = (uint32_t)v[1], w2 = (uint32_t)v[2], w3 = (uint32_t)v[3];
+  return v4i{(int)__builtin_amdgcn_perm(w1, w0, 0x05040100u), (int)__builtin_amdgcn_perm(w3, w2, 0x05040100u),
+             (int)__builtin_amdgcn_perm(w1, w0, 0x07060302u), (int)__builtin_amdgcn_perm(w3, w2, 0x07060302u)};
+}
+
+// a pointer the caller knows to be wave-uniform, as SGPRs
+__device__ __forceinline__ const uint8_t* uniform_ptr(const uint8_t* p) {
+  const uint64_t v = reinterpret_cast<uint64_t>(p);
+  const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v), hi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
+  return reinterpret_cast<const uint8_t*>(((uint64_t)hi << 32) | lo);
+}
+
+// s_waitcnt immediates (gfx9 encoding: vmcnt [3:0] and [15:14], expcnt [6:4],
+// lgkmcnt [11:8]; an all-ones field does not wait): vmcnt <= n (n < 64) alone;
+// every LDS read returned
+constexpr int vmcnt_at_most(int n) { return ((n >> 4) << 14) | 0x0F70 | (n & 15); }
+constexpr int kLdsRead = 0xC07F;
+
 template <int kWidth>
 __device__ __forceinline__ float reduce_max_xor(float v) {
 #pragma unroll

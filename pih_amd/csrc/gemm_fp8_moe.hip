@@ -72,19 +72,9 @@ constexpr uint32_t smem_bytes() {
 }
 constexpr int kWaitVm0 = 0x0F70;     // vmcnt(0)
 constexpr uint32_t kCodePitch = 144;  // staged e4m3 code rows (128 bytes + 16)
-// s_waitcnt immediate waiting for vmcnt <= n (n < 64; bits [3:0] and [15:14])
-constexpr int vmcnt_enc(int n) { return ((n >> 4) << 14) | 0x0F70 | (n & 15); }
-static_assert(vmcnt_enc(7) == kWaitVm7 && vmcnt_enc(0) == kWaitVm0, "vmcnt encoding");
+static_assert(vmcnt_at_most(7) == kWaitVm7 && vmcnt_at_most(0) == kWaitVm0, "vmcnt encoding");
 // stores one lane of a persistent block issues per tile of plain output
 constexpr uint32_t kStoreOps = 16;
-
-// LDS byte address of a __shared__ object
-// a pointer the caller knows to be wave-uniform, as SGPRs
-__device__ __forceinline__ const uint8_t* uniform_ptr(const uint8_t* p) {
-  const uint64_t v = reinterpret_cast<uint64_t>(p);
-  const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v), hi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
-  return reinterpret_cast<const uint8_t*>(((uint64_t)hi << 32) | lo);
-}
 
 // byte offset of 16-byte chunk c of tile row r (XOR-swizzled slots)
 __device__ __forceinline__ uint32_t lds_at(uint32_t r, uint32_t c) { return r * LDS_ROW + ((c ^ ((r >> 1) & 7u)) << 4); }
@@ -976,8 +966,8 @@ __global__ __launch_bounds__(NTH, 1) void fp8_moe_gemm_kernel(MoeParams p) {
   // scales 1 (bf16: 0)
   constexpr int kLoads = kBf ? 6 : kF4 ? 5 : 7;
   static_assert(kLoads == kNLoads, "loads per step");
-  constexpr int kWaitStep = vmcnt_enc((int)(NS - 2) * kLoads);
-  constexpr int kWaitFirstEnc = vmcnt_enc(kLoads + (int)kStoreOps);
+  constexpr int kWaitStep = vmcnt_at_most((int)(NS - 2) * kLoads);
+  constexpr int kWaitFirstEnc = vmcnt_at_most(kLoads + (int)kStoreOps);
   // stages of steps kb + 0, 1, 2 (kb a multiple of 3)
   const uint32_t st0 = rot, st1 = rot == 2 ? 0u : rot + 1, st2 = rot == 0 ? 2u : rot - 1;
   // persistent blocks run steps 0 .. KB - 3 in the unrolled loop and the

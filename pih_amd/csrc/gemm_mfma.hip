@@ -187,12 +187,6 @@ __device__ __forceinline__ v8i cat8(v4i x, v4i y) {
   return v8i{x[0], x[1], x[2], x[3], y[0], y[1], y[2], y[3]};
 }
 
-__device__ __forceinline__ uint32_t ff_bytes(uint32_t w) {
-  // non-zero when any byte of w is 0xFF
-  const uint32_t n = ~w;
-  return (n - 0x01010101u) & ~n & 0x80808080u;
-}
-
 // An operand fragment whose E8M0 block scale is 0xFF (the reference skips
 // that block) becomes zeros with scale 127, so its products add exactly 0;
 // the test is wave-wide, and the select runs only in a wave that has one.

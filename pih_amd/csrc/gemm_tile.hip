@@ -70,17 +70,6 @@ struct TileParams {
 
 typedef unsigned int v4u __attribute__((ext_vector_type(4)));
 
-__device__ __forceinline__ const uint8_t* uniform_ptr(const uint8_t* p) {
-  const uint64_t v = reinterpret_cast<uint64_t>(p);
-  const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v), hi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
-  return reinterpret_cast<const uint8_t*>(((uint64_t)hi << 32) | lo);
-}
-
-// s_waitcnt immediates: vmcnt <= n (n < 64) alone; every LDS read returned
-// (the stage a wave has read may be refilled once all are past the barrier)
-constexpr int vmcnt_at_most(int n) { return ((n >> 4) << 14) | 0x0F70 | (n & 15); }
-constexpr int kLdsRead = 0xC07F;
-
 // Output element (A row ar, column col of problem prob) the reference's way,
 // by a whole wave (every lane the same element): per 128-k block an fp32 sum
 // of decoded e4m3 products in k order with NaN codes as 0, the blocks added
@@ -185,8 +174,6 @@ __device__ __forceinline__ v4f without_ff_block(uint32_t ws, uint32_t as, v4f be
   return v4f{skip ? before[0] : after[0], skip ? before[1] : after[1], skip ? before[2] : after[2],
              skip ? before[3] : after[3]};
 }
-
-__device__ __forceinline__ uint32_t has_ff(uint32_t v) { return (~v - 0x01010101u) & v & 0x80808080u; }
 
 template <int OP, int MB, int NB>
 struct TileShape {
@@ -341,7 +328,8 @@ __global__ __launch_bounds__(kThreads, 1) void tile_gemm_kernel(TileParams p) {
   // ---- the K loop: ST stages.  A loading wave waits for its part of step
   // j's stage, meets the others at the barrier and sends for step j + ST - 1
   // (the last ST - 1 steps send for nothing and wait for less each); a
-  // multiplying wave meets the barrier and multiplies step j.
+  // multiplying wave waits for its own LDS reads (the stage it has read may be
+  // refilled once all are past the barrier), meets it and multiplies step j.
   const uint32_t lead = min((uint32_t)(ST - 1), steps);
   auto tail_wait = [&](int left) __attribute__((always_inline)) {
     // `left` further steps are in flight
@@ -426,9 +414,9 @@ __global__ __launch_bounds__(kThreads, 1) void tile_gemm_kernel(TileParams p) {
       uint32_t hit = 0;
       for (uint32_t i = lane; i < TM * KB / 16; i += 64) {
         const v4u v = reinterpret_cast<const v4u*>(pa)[i];
-        hit |= has_ff(v.x) | has_ff(v.y) | has_ff(v.z) | has_ff(v.w);
+        hit |= ff_bytes(v.x) | ff_bytes(v.y) | ff_bytes(v.z) | ff_bytes(v.w);
       }
-      if (lane < KB / 4) hit |= has_ff(reinterpret_cast<const uint32_t*>(pw)[lane]);
+      if (lane < KB / 4) hit |= ff_bytes(reinterpret_cast<const uint32_t*>(pw)[lane]);
       ff = __builtin_amdgcn_ballot_w64(hit != 0) != 0;
       if (ff) bad |= kErrScale;
     }
@@ -734,9 +722,9 @@ __global__ __launch_bounds__(kThreads, 1) void tile_grid_kernel(TileParams p) {
       uint32_t hit = 0;
       for (uint32_t e = lane; e < TM * KB / 16; e += 64) {
         const v4u v = reinterpret_cast<const v4u*>(pan + 256)[e];
-        hit |= has_ff(v.x) | has_ff(v.y) | has_ff(v.z) | has_ff(v.w);
+        hit |= ff_bytes(v.x) | ff_bytes(v.y) | ff_bytes(v.z) | ff_bytes(v.w);
       }
-      if (lane < KB / 4) hit |= has_ff(reinterpret_cast<const uint32_t*>(pan)[lane]);
+      if (lane < KB / 4) hit |= ff_bytes(reinterpret_cast<const uint32_t*>(pan)[lane]);
       ff = __builtin_amdgcn_ballot_w64(hit != 0) != 0;
       if (ff) bad |= kErrScale;
     }

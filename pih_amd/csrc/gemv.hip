@@ -290,28 +290,6 @@ __device__ __forceinline__ v4i nt_piece(const void* w, uint64_t elem_offset) {
     return __builtin_nontemporal_load(reinterpret_cast<const v4i*>(static_cast<const uint32_t*>(w) + elem_offset));
 }
 
-// 8 nibbles of one word (nibble j = k offset j) -> eight bf16 values
-// 128 + u_j in the order k = 0, 2, 4, 6, 1, 3, 5, 7: the low nibbles of the
-// four bytes are the even k, the high nibbles the odd k, and one v_perm per
-// pair places two of them under the 0x43 exponent byte of 128.  x is staged
-// in LDS in the same order (x_in_nibble_order), so the MFMA sees matching
-// k on both operands.
-__device__ __forceinline__ void nibbles_to_bf16(uint32_t w, v4i& out) {
-  const uint32_t lo = w & 0x0F0F0F0Fu, hi = (w >> 4) & 0x0F0F0F0Fu;
-  constexpr uint32_t kExp = 0x43434343u;
-  out[0] = (int)__builtin_amdgcn_perm(kExp, lo, 0x04010400u);  // k0, k2
-  out[1] = (int)__builtin_amdgcn_perm(kExp, lo, 0x04030402u);  // k4, k6
-  out[2] = (int)__builtin_amdgcn_perm(kExp, hi, 0x04010400u);  // k1, k3
-  out[3] = (int)__builtin_amdgcn_perm(kExp, hi, 0x04030402u);  // k5, k7
-}
-
-// Eight bf16 x values (k = 0..7) into the order nibbles_to_bf16 produces.
-__device__ __forceinline__ v4i x_in_nibble_order(v4i v) {
-  const uint32_t w0 = (uint32_t)v[0], w1 = (uint32_t)v[1], w2 = (uint32_t)v[2], w3 = (uint32_t)v[3];
-  return v4i{(int)__builtin_amdgcn_perm(w1, w0, 0x05040100u), (int)__builtin_amdgcn_perm(w3, w2, 0x05040100u),
-             (int)__builtin_amdgcn_perm(w1, w0, 0x07060302u), (int)__builtin_amdgcn_perm(w3, w2, 0x07060302u)};
-}
-
 // U consecutive 16-bit scales of one row, starting at a multiple of U.
 template <int U>
 struct ScaleVec {
@@ -544,7 +522,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemv_lds_kernel(GemvGroup grp, uin
         }
         v4i qb[4];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) nibbles_to_bf16(wd[i], qb[i]);
+        for (int i = 0; i < 4; ++i) qb[i] = nibbles_to_bf16(wd[i]);
         v4f pq = v4f{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int i = 0; i < 4; ++i)
@@ -787,7 +765,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemv_mid_kernel(GemvGroup grp, uin
             }
             v4i qb[4];
 #pragma unroll
-            for (int i = 0; i < 4; ++i) nibbles_to_bf16(wd[i], qb[i]);
+            for (int i = 0; i < 4; ++i) qb[i] = nibbles_to_bf16(wd[i]);
             const float zc = 128.0f + (float)zero;
 #pragma unroll
             for (int t = 0; t < MT; ++t) {

@@ -94,12 +94,6 @@ __device__ __forceinline__ v8i cat8(v4i x, v4i y) {
   return v8i{x[0], x[1], x[2], x[3], y[0], y[1], y[2], y[3]};
 }
 
-// non-zero when any byte of w is 0xFF (a NaN UE8M0 scale)
-__device__ __forceinline__ uint32_t ff_bytes(uint32_t w) {
-  const uint32_t n = ~w;
-  return (n - 0x01010101u) & ~n & 0x80808080u;
-}
-
 // Block -> (expert, first row, rows, W block) over the light experts only
 // (1 <= rows <= kMoeLightRows).  An expert with more than max_rows rows is
 // done in ceil(rows / max_rows) row chunks; items are numbered expert-major,

@@ -48,28 +48,6 @@ struct W4Params {
   uint32_t m, k, count, tiles;
 };
 
-__device__ __forceinline__ const uint8_t* uniform_ptr(const uint8_t* p) {
-  const uint64_t v = reinterpret_cast<uint64_t>(p);
-  const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v), hi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
-  return reinterpret_cast<const uint8_t*>(((uint64_t)hi << 32) | lo);
-}
-constexpr int vmcnt_at_most(int n) { return ((n >> 4) << 14) | 0x0F70 | (n & 15); }
-constexpr int kLdsRead = 0xC07F;
-
-// eight nibbles -> bf16 128 + u in the order k 0, 2, 4, 6, 1, 3, 5, 7
-__device__ __forceinline__ v4i nibbles_to_bf16(uint32_t w) {
-  const uint32_t lo = w & 0x0F0F0F0Fu, hi = (w >> 4) & 0x0F0F0F0Fu;
-  constexpr uint32_t kExp = 0x43434343u;
-  return v4i{(int)__builtin_amdgcn_perm(kExp, lo, 0x04010400u), (int)__builtin_amdgcn_perm(kExp, lo, 0x04030402u),
-             (int)__builtin_amdgcn_perm(kExp, hi, 0x04010400u), (int)__builtin_amdgcn_perm(kExp, hi, 0x04030402u)};
-}
-// eight bf16 x values into that order
-__device__ __forceinline__ v4i x_in_nibble_order(v4i v) {
-  const uint32_t w0 = (uint32_t)v[0], w1 = (uint32_t)v[1], w2 = (uint32_t)v[2], w3 = (uint32_t)v[3];
-  return v4i{(int)__builtin_amdgcn_perm(w1, w0, 0x05040100u), (int)__builtin_amdgcn_perm(w3, w2, 0x05040100u),
-             (int)__builtin_amdgcn_perm(w1, w0, 0x07060302u), (int)__builtin_amdgcn_perm(w3, w2, 0x07060302u)};
-}
-
 // XI x rows a loading wave moves per step: 4 XI rows in all, whole 16-row MFMA
 // operands
 template <int XI, int NB>
